@@ -239,7 +239,7 @@ struct mspai_ctx {
     int nb = 0, maxbs = 1, bcmax = 0, brmax = 0;
     long long nnzb = 0;
     std::vector<int> h_bsize, h_bcolptr, h_browind;
-    int *d_bsize = nullptr, *d_bstart = nullptr, *d_bcolptr = nullptr, *d_browind = nullptr;
+    int *d_bsize = nullptr, *d_bstart = nullptr, *d_bmap = nullptr, *d_bcolptr = nullptr, *d_browind = nullptr;
     int *d_brp_ptr = nullptr, *d_brp_ind = nullptr;
     long long *d_bvoff = nullptr, *d_sqoff = nullptr;
     double *d_bval = nullptr, *d_sqinv = nullptr, *d_sqtmp = nullptr;
@@ -283,6 +283,7 @@ static void block_free(mspai_ctx* ctx)
 {
     dfree(ctx->d_bsize);
     dfree(ctx->d_bstart);
+    dfree(ctx->d_bmap);
     dfree(ctx->d_bcolptr);
     dfree(ctx->d_browind);
     dfree(ctx->d_brp_ptr);
@@ -308,6 +309,7 @@ static void block_free(mspai_ctx* ctx)
 }
 
 static int block_convert(mspai_ctx* ctx);
+static int block_values(mspai_ctx* ctx);
 
 extern "C" void mspai_default_opts(mspai_opts* o)
 {
@@ -572,11 +574,12 @@ extern "C" int mspai_update_values(mspai_ctx* ctx, const double* val)
     if (!ctx || !val || !ctx->d_val) return MSPAI_ERR_ARG;
     HIPCHK(hipSetDevice(ctx->device));
     HIPCHK(hipMemcpyAsync(ctx->d_val, val, ctx->nnz * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
     ctx->nnzM = -1;
     ctx->mixed_fp64_last = -1;
     ctx->a_csr_ok = ctx->m_csr_ok = ctx->ajn_ok = false;
-    if (ctx->block_bs != 1) return block_convert(ctx);  // Convert_Block_Matrix_Update
+    int rc;
+    if (ctx->block_bs != 1 && (rc = block_values(ctx))) return rc;  // Convert_Block_Matrix_Update
+    HIPCHK(hipStreamSynchronize(ctx->stream));
     return MSPAI_OK;
 }
 
@@ -1599,11 +1602,12 @@ extern "C" int mspai_update_values_device(mspai_ctx* ctx, const double* d_val)
     if (!ctx || !d_val || !ctx->d_val) return MSPAI_ERR_ARG;
     HIPCHK(hipSetDevice(ctx->device));
     HIPCHK(hipMemcpyAsync(ctx->d_val, d_val, ctx->nnz * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
     ctx->nnzM = -1;
     ctx->mixed_fp64_last = -1;
     ctx->a_csr_ok = ctx->m_csr_ok = ctx->ajn_ok = false;
-    if (ctx->block_bs != 1) return block_convert(ctx);
+    int rc;
+    if (ctx->block_bs != 1 && (rc = block_values(ctx))) return rc;
+    HIPCHK(hipStreamSynchronize(ctx->stream));
     return MSPAI_OK;
 }
 
@@ -2097,6 +2101,7 @@ static int block_convert(mspai_ctx* ctx)
     int rc;
     if ((rc = upload(ctx, ctx->d_bsize, ctx->h_bsize.data(), nb))) return rc;
     if ((rc = upload(ctx, ctx->d_bstart, start.data(), nb + 1))) return rc;
+    if ((rc = upload(ctx, ctx->d_bmap, bmap.data(), n))) return rc;
     if ((rc = upload(ctx, ctx->d_bcolptr, bcp.data(), nb + 1))) return rc;
     if ((rc = upload(ctx, ctx->d_browind, bri.data(), bri.size()))) return rc;
     if ((rc = upload(ctx, ctx->d_bvoff, voff.data(), voff.size()))) return rc;
@@ -2112,6 +2117,22 @@ static int block_convert(mspai_ctx* ctx)
     ctx->bcmax = bcmax;
     ctx->brmax = brmax;
     ctx->nnzb = nnzb;
+    return MSPAI_OK;
+}
+
+/* New values of A on the pattern block_convert laid out: the blocks' zeros
+ * stay, every stored scalar entry goes to its place in its block. */
+static int block_values(mspai_ctx* ctx)
+{
+    BlockArgs a{};
+    a.bsize = ctx->d_bsize;
+    a.bstart = ctx->d_bstart;
+    a.colptr = ctx->d_bcolptr;
+    a.rowind = ctx->d_browind;
+    a.voff = ctx->d_bvoff;
+    const DevCsc A{ctx->nrows, ctx->ncols, ctx->d_colptr, ctx->d_rowind, ctx->d_val};
+    launch_block_values(a, A, ctx->d_bmap, ctx->d_bval, ctx->stream);
+    HIPCHK(hipGetLastError());
     return MSPAI_OK;
 }
 

@@ -550,6 +550,30 @@ __global__ __launch_bounds__(64, 4) void block_column_kernel(BlockArgs a, BlockL
     }
 }
 
+/* Convert_Block_Matrix_Update: the values of A's stored entries to their
+ * places in the blocks (entry (i, j) of block (ib, jb) at voff + (j -
+ * start_jb) h + i - start_ib).  kValueLanes lanes per scalar column, one
+ * entry each per round, so that a column's row indices and values are read
+ * together; the block is found by a binary search of the block column (a
+ * few entries).  Bound by the scattered 8 B stores; the pattern does not
+ * change with the values, so neither the offsets nor the blocks' zeros are
+ * rebuilt. */
+constexpr int kValueLanes = 8;
+
+__global__ __launch_bounds__(256) void block_values_kernel(BlockArgs a, DevCsc A, const int* bmap, double* bval)
+{
+    const int j = blockIdx.x * (256 / kValueLanes) + (int)threadIdx.x / kValueLanes;
+    if (j >= A.ncols) return;
+    const int jb = bmap[j], dc = j - a.bstart[jb];
+    const int b0 = a.colptr[jb], nbr = a.colptr[jb + 1] - b0;
+    const int end = A.colptr[j + 1];
+    for (int e = A.colptr[j] + (int)threadIdx.x % kValueLanes; e < end; e += kValueLanes) {
+        const int i = A.rowind[e], ib = bmap[i];
+        const int t = lower_bound_i(a.rowind + b0, nbr, ib);
+        bval[a.voff[b0 + t] + (long long)dc * a.bsize[ib] + (i - a.bstart[ib])] = A.val[e];
+    }
+}
+
 /* Compute_Square_Inverse for every block column: S = A_j^T A_j by
  * Mult_Blocks_TN over the stored blocks (unfused, storage order), then S^-1
  * by Gauss-Jordan elimination with partial pivoting (first largest |pivot|),
@@ -651,6 +675,14 @@ __global__ void block_scalar_fill_kernel(BlockArgs a, const int* colptr, int* ro
 }
 
 }  // namespace
+
+void launch_block_values(const BlockArgs& a, const DevCsc& A, const int* bmap, double* bval, hipStream_t stream)
+{
+    constexpr int kCols = 256 / kValueLanes;
+    if (A.ncols <= 0) return;
+    hipLaunchKernelGGL(block_values_kernel, dim3((A.ncols + kCols - 1) / kCols), dim3(256), 0, stream, a, A, bmap,
+                       bval);
+}
 
 void launch_block_sq_inverse(const BlockArgs& a, double* tmp, hipStream_t stream)
 {

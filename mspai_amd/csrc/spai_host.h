@@ -52,6 +52,9 @@ void launch_line_dot(int nlines, const int* ptr, const int* ind, const double* v
                      hipStream_t stream);
 
 /* Block SPAI (spai_block.hip). */
+/* Values of A's stored entries into the blocks (a: sizes, offsets and the block
+ * pattern; bmap: scalar index -> block). */
+void launch_block_values(const BlockArgs& a, const DevCsc& A, const int* bmap, double* bval, hipStream_t stream);
 /* (A_j^T A_j)^-1 of every block column into a.sqinv (tmp: sum bsize^2 doubles). */
 void launch_block_sq_inverse(const BlockArgs& a, double* tmp, hipStream_t stream);
 /* Persistent block-column kernel on nwaves waves, L.per_wave bytes each at a.scratch. */

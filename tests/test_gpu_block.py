@@ -161,6 +161,31 @@ def test_block_reuse_pattern_and_new_values(blk, gpu):
     assert same_csc_bitwise(blk.to_scalar(B2, ref), M2)
 
 
+@pytest.mark.parametrize("size,fields,bs", [(7, 3, 2), (7, 3, 4), (6, 2, 0), (1, 3, 3), (8, 3, 6)])
+def test_block_values_from_device(blk, gpu, size, fields, bs):
+    """New values from device memory after a first build (blocks that do not
+    divide n, blocks of varying size, a single block, columns with more than
+    eight entries): the adaptive build equals the oracle's on the new matrix,
+    bit for bit."""
+    A = gen.block_convdiff2d(size, fields, seed=21)
+    rng = np.random.Generator(np.random.PCG64(22))
+    A2 = A.copy()
+    A2.data = A2.data * (1.0 + 0.05 * rng.standard_normal(A2.nnz))
+    b = gpu.Builder(0)
+    try:
+        b.upload(A)
+        b.set_block_size(bs)
+        b.build(**ADAPT)
+        v = torch.tensor(A2.data, device="cuda")
+        b.update_values_device(v.data_ptr())
+        b.build(**ADAPT)
+        M = b.download()
+    finally:
+        b.close()
+    B = blk.BlockMatrix(A2, _sizes(blk, A, bs))
+    assert same_csc_bitwise(blk.to_scalar(B, blk.spai_block(B, None, threads=16, **ADAPT)), M)
+
+
 def test_block_apply_and_back_to_scalar(blk, gpu, oracle):
     """M of a block build applies like scipy's product; bs = 1 returns to the
     scalar path (bitwise equal to the scalar oracle)."""
