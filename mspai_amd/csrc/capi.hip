@@ -160,6 +160,8 @@ struct mspai_ctx {
     // start pattern
     int *d_p_ptr = nullptr, *d_p_ind = nullptr;
     int plen_max = 0;
+    int p_nnz = 0;              // entries of the start pattern
+    bool p_base0 = true;        // its colptr starts at 0
     int p_cols = 0;             // columns the start pattern was set for
     int *d_up_ptr = nullptr, *d_up_ind = nullptr;  // upper pattern (-up), CSC; nullptr: none
     int up_cols = 0;
@@ -201,7 +203,7 @@ struct mspai_ctx {
     int* d_csr_tmp = nullptr;  // 4 x csr_tmp_cap ints: columns, order, sorted rows, permutation
     long long csr_tmp_cap = 0;
     bool a_csr_ok = false, m_csr_ok = false;
-    bool ajn_ok = false;  // d_ajn holds the column norms of the current values
+    bool ajn_ok = false;  // d_ajn (and d_rp_val) hold the column norms (row values) of the current values
     hipEvent_t ev[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};  // [4..5]: first size bin
     hipEvent_t csr_ev = nullptr;  // orders a CSR copy on the context's stream with the caller's stream
     /* per-launch profile of the last build: events around every column-kernel
@@ -614,6 +616,8 @@ extern "C" int mspai_set_pattern(mspai_ctx* ctx, const int* colptr, const int* r
     if ((rc = upload(ctx, ctx->d_p_ind, rowind, (size_t)colptr[n]))) return rc;
     HIPCHK(hipStreamSynchronize(ctx->stream));
     ctx->plen_max = pmax;
+    ctx->p_nnz = colptr[n];
+    ctx->p_base0 = colptr[0] == 0;
     ctx->p_cols = n;
     ctx->pattern_set = true;
     return MSPAI_OK;
@@ -1097,7 +1101,7 @@ static int begin_launch(mspai_ctx* ctx, BuildArgs& a, const char* what, int mode
 {
     const int k = ctx->nlaunch;
     if (k >= kMaxLaunch) return fail(ctx, MSPAI_ERR_STATE, "more column-kernel launches than the profile holds");
-    static const char* kModes[] = {"FP64", "mixed", "adjoint FP64", "adjoint mixed", "FP64 QR update"};
+    static const char* kModes[] = {"FP64", "mixed", "adjoint", "", "FP64 QR update"};
     if (b)
         std::snprintf(ctx->lname[k], sizeof ctx->lname[k], "%s bin %d G=%d |J|<=%d |I|<=%d", kModes[mode], bin,
                       b->group, b->L.capJ, b->L.capI);
@@ -1125,7 +1129,7 @@ static size_t tie_bytes_needed(const mspai_ctx* ctx, const std::vector<Bin>& bin
         need = std::max(need, (size_t)ctx->num_cu * waves_per_cu(b, fp64_mode) * (64 / b.group) * b.L.tie_per_group);
     if (mixed)
         for (const Bin& b : bins)
-            need = std::max(need, (size_t)ctx->num_cu * waves_per_cu(b, b.fp64 ? fp64_mode : (fp64_mode == 2 ? 3 : 1)) *
+            need = std::max(need, (size_t)ctx->num_cu * waves_per_cu(b, b.fp64 ? fp64_mode : 1) *
                                       (64 / b.group) * b.L.tie_per_group);
     return need;
 }
@@ -1208,7 +1212,7 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
             a.n_overflow = b + 1 < nb ? mcounts + b + 1 : counts + to;
             /* a bin the table runs in FP64 inside the mixed chain passes its
              * overflow on like the others and declines nothing */
-            const int mode = bins[b].fp64 ? fp64_mode : (fp64_mode == 2 ? 3 : 1);
+            const int mode = bins[b].fp64 ? fp64_mode : 1;
             int per_cu = waves_per_cu(bins[b], mode);
             const ScratchLayout& L = bins[b].L;
             if (b == 0) HIPCHK(hipEventRecord(ctx->ev[4], ctx->stream));
@@ -1264,6 +1268,108 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
     if ((rc = end_launch(ctx))) return rc;
     if (nf == 0) HIPCHK(hipEventRecord(ctx->ev[5], ctx->stream));
     return MSPAI_OK;
+}
+
+/* The bins of static builds and the adjoint: the kinds of the given-pattern
+ * kernels, then one 64-lane LDS bin of |J| <= 40, |I| <= 128 for the wider
+ * columns (`wide`: its layout, none when the kinds hold every column), then
+ * the generic kernel. */
+static std::vector<Bin> static_wide_bin(const mspai_ctx* ctx, int cap, const ScratchLayout& G, int needs)
+{
+    static const BinTable kWide = {"g64", 1, {{64, 40, 128, 512, 1024, 0}}};
+    return bin_layouts(ctx, cap, 1, false, G, kWide, needs);
+}
+
+/* Launch a static build (mode 0) or the adjoint (mode 2) over the columns
+ * whose patterns are in a.p_ptr/p_ind, at most `longest` and on average
+ * `mean` entries long.  When one kind holds the longest column and the
+ * average column is at least half as long, the kind takes all columns by
+ * index and the routing kernel is not run (71 to 120 us of 0.26 million
+ * columns); lists of more uneven columns are routed, so that short ones run
+ * eight to a wave.  *first: that kind, or -1.  Queues and counters as in
+ * run_chain, queue b < kStaticKinds for the kinds, then the wide bin's, then
+ * the generic kernel's. */
+static int run_static(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& wide, const ScratchLayout& G, int gwaves,
+                      int mode, bool refine, int n, int longest, double mean, int* first)
+{
+    const bool back = mode == 2;
+    const int nf = kStaticKinds + (int)wide.size();
+    int* counts = ctx->d_counter;
+    int* heads = ctx->d_counter + 8;
+    int* q = ctx->d_queues;
+    int rc;
+    launch_fill_int(ctx->d_counter, 64, 0, ctx->stream);  // a kernel, not a memset node
+    HIPCHK(hipGetLastError());
+    ctx->nlaunch = 0;
+    ctx->lwork_valid = false;
+    a.status_or = 0;
+    a.save_state = 0;
+    const size_t tie_need = tie_bytes_needed(ctx, wide, wide, false, mode);
+    if (tie_need > ctx->tie_bytes) {
+        if (ctx->no_alloc) return fail(ctx, MSPAI_ERR_CAPACITY, "tie buffers: this call allocates no device memory");
+        dfree(ctx->d_tie);
+        HIPCHK(hipMalloc((void**)&ctx->d_tie, tie_need));
+        ctx->tie_bytes = tie_need;
+    }
+    a.tie_scratch = ctx->d_tie;
+    int kind = 0;
+    while (kind < kStaticKinds && kStaticJ[kind] < longest) ++kind;
+    *first = kind < kStaticKinds && (kind == 0 || 2.0 * mean >= longest) ? kind : -1;
+    if (*first < 0) {
+        BinEdges edges{};
+        for (int b = 0; b < kStaticKinds; ++b) {
+            edges.capJ[b] = kStaticJ[b];
+            edges.capI[b] = kStaticI[b];
+            edges.capSort[b] = 0x7fffffff;
+        }
+        for (const Bin& b : wide) {
+            edges.capJ[kStaticKinds] = b.L.capJ;
+            edges.capI[kStaticKinds] = b.L.capI;
+            edges.capSort[kStaticKinds] = b.L.capSid;
+        }
+        launch_classify(a, nf, edges, q, counts, q + (size_t)nf * n, counts + nf, n, ctx->d_counter + 40,
+                        ctx->d_counter + 16, ctx->stream);
+        HIPCHK(hipGetLastError());
+    }
+    HIPCHK(hipEventRecord(ctx->ev[4], ctx->stream));
+    bool all_fit = false;
+    for (int b = std::max(*first, 0); b < kStaticKinds && !all_fit; ++b) {
+        /* past the kind that takes every column, only one with room for more rows */
+        if (*first >= 0 && b > *first && kStaticI[b] <= kStaticI[b - 1]) continue;
+        /* a column moves on to the next kind with more rows */
+        int next = b + 1;
+        while (next < kStaticKinds && kStaticI[next] <= kStaticI[b]) ++next;
+        a.overflow = q + (size_t)next * n;
+        a.n_overflow = counts + next;
+        char what[40];
+        std::snprintf(what, sizeof what, "given pattern |J|<=%d |I|<=%d", kStaticJ[b], kStaticI[b]);
+        if ((rc = begin_launch(ctx, a, what, mode, -1, nullptr))) return rc;
+        const bool direct = b == *first;
+        launch_static_columns(b, a, back, refine, direct ? nullptr : q + (size_t)b * n, counts + b, n, ctx->num_cu,
+                              ctx->stream);
+        HIPCHK(hipGetLastError());
+        if ((rc = end_launch(ctx))) return rc;
+        if (b == std::max(*first, 0)) HIPCHK(hipEventRecord(ctx->ev[5], ctx->stream));
+        /* no column of the pattern can have more rows than this kind takes */
+        all_fit = direct && (size_t)longest * ctx->maxcolnnz <= (size_t)kStaticI[b];
+    }
+    if (all_fit) return MSPAI_OK;
+    for (int b = 0; b < (int)wide.size(); ++b) {
+        const int t = kStaticKinds + b;
+        a.overflow = q + (size_t)(t + 1) * n;
+        a.n_overflow = counts + t + 1;
+        if ((rc = begin_launch(ctx, a, nullptr, mode, t, &wide[b]))) return rc;
+        launch_binned(a, wide[b].L, wide[b].group, mode, q + (size_t)t * n, counts + t, heads + t,
+                      ctx->num_cu * waves_per_cu(wide[b], mode), ctx->stream, wide[b].wcap);
+        HIPCHK(hipGetLastError());
+        if ((rc = end_launch(ctx))) return rc;
+    }
+    a.overflow = q;  // never written: the generic layout holds every column
+    a.n_overflow = counts + 7;
+    if ((rc = begin_launch(ctx, a, "generic (HBM working set)", mode, -1, nullptr))) return rc;
+    launch_fp64_generic(a, G, mode, q + (size_t)nf * n, counts + nf, heads + nf, gwaves, ctx->stream);
+    HIPCHK(hipGetLastError());
+    return end_launch(ctx);
 }
 
 /* Queue the copy of the counters to the pinned host array (after the last
@@ -1340,6 +1446,13 @@ static int prepare_generic(mspai_ctx* ctx, const ScratchLayout& G, int* gwaves)
     return ensure_scratch(ctx, (size_t)w * G.per_wave);
 }
 
+/* A static build with size bins that keeps neither counters nor the cache. */
+static bool given_pattern_build(const mspai_ctx* ctx, const mspai_opts* o)
+{
+    return o->max_impr_steps == 0 && o->binning && !o->counters && !(o->cache > 0 && o->precision == 0) &&
+           !ctx->d_up_ptr && ctx->p_base0;
+}
+
 static BuildArgs base_args(mspai_ctx* ctx)
 {
     BuildArgs a{};
@@ -1379,7 +1492,14 @@ extern "C" int mspai_build(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* 
     const int needs = (qrup ? kNeedQrUpdate : 0) | (opts->precision == 1 && !qrup ? kNeedMixed : 0);
     const ScratchLayout G = generic_layout(ctx, cap, opts->maxnew, adaptive, needs);
     std::vector<Bin> bins, fbins;
-    if (opts->binning && !ctx->d_up_ptr) {  // an upper pattern runs unbinned
+    /* static builds take the given-pattern kernels, FP64 under either
+     * precision, whatever the bin table (not with counters or the cache,
+     * which only the adaptive builds' kernels keep) */
+    const bool given = given_pattern_build(ctx, opts);
+    if (given) {
+        bins = static_wide_bin(ctx, cap, G, needs & ~kNeedMixed);
+        ctx->last_table = table_for(ctx, opts);
+    } else if (opts->binning && !ctx->d_up_ptr) {  // an upper pattern runs unbinned
         int t = table_for(ctx, opts);
         bins = bin_layouts(ctx, cap, opts->maxnew, adaptive, G, kTables[t], needs);
         /* the FP64 chain of a mixed build: the same table in FP64 layouts
@@ -1394,7 +1514,7 @@ extern "C" int mspai_build(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* 
 
     HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
     BuildArgs a = base_args(ctx);
-    if (!ctx->ajn_ok) {  // once per set of values
+    if (adaptive && !ctx->ajn_ok) {  // once per set of values; only the candidate scores read them
         hipLaunchKernelGGL(column_norms_kernel, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, a.A, ctx->d_ajn);
         if (a.rp_val)
             hipLaunchKernelGGL(row_values_kernel, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, a.A, a.rp_ptr,
@@ -1418,7 +1538,12 @@ extern "C" int mspai_build(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* 
     a.nsolve = ctx->d_nsolve;
     a.status = ctx->d_status;
     a.work = opts->counters ? ctx->d_work : nullptr;  // opt-in: 64 B per column of writes
-    const bool mixed = opts->precision == 1 && !bins.empty() && !qrup;
+    const bool mixed = opts->precision == 1 && !bins.empty() && !qrup && !given;
+    if (given) {
+        a.direct = 1;
+        a.m_idx = ctx->d_Mind;
+        a.m_val = ctx->d_Mval;
+    }
     if (opts->cache > 0 && !qrup && opts->precision == 0) {
         const int cI = std::min(G.capI, 32), cJ = std::min(cap, 16);
         if ((rc = ensure_cache(ctx, opts->cache, cI, cJ))) return rc;
@@ -1435,17 +1560,27 @@ extern "C" int mspai_build(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* 
         a.cache_hits = ctx->d_counter + 48;
     }
     HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
-    if ((rc = run_chain(ctx, a, bins, fbins, G, gwaves, mixed, qrup ? 4 : 0, n))) return rc;
+    int first = -1;
+    if (given) {
+        if ((rc = run_static(ctx, a, bins, G, gwaves, 0, opts->precision == 1, n, ctx->plen_max, (double)ctx->p_nnz / n, &first))) return rc;
+    } else {
+        if ((rc = run_chain(ctx, a, bins, fbins, G, gwaves, mixed, qrup ? 4 : 0, n))) return rc;
+    }
     HIPCHK(hipEventRecord(ctx->ev[2], ctx->stream));
 
-    /* compaction: colptr[0] = 0, colptr[1..n] = inclusive scan of the lengths */
-    size_t cub_bytes = ctx->cub_bytes;
-    HIPCHK(hipcub::DeviceScan::InclusiveSum(ctx->d_cub, cub_bytes, ctx->d_m_len, ctx->d_Mptr + 1, n,
-                                             ctx->stream));
-    constexpr int kScatterCols = 256 / kScatterLanes;
-    hipLaunchKernelGGL(scatter_columns_kernel, dim3((n + kScatterCols - 1) / kScatterCols), dim3(256), 0,
-                       ctx->stream, n, cap, ctx->d_m_len, ctx->d_m_idx, ctx->d_m_val, ctx->d_Mptr, ctx->d_Mind,
-                       ctx->d_Mval, ctx->d_counter + 63);
+    if (given) {
+        launch_copy_pattern(n, ctx->p_nnz, ctx->d_p_ptr, ctx->d_p_ind, ctx->d_Mptr, ctx->d_Mind,
+                            ctx->d_counter + 63, ctx->stream);
+    } else {
+        /* compaction: colptr[0] = 0, colptr[1..n] = inclusive scan of the lengths */
+        size_t cub_bytes = ctx->cub_bytes;
+        HIPCHK(hipcub::DeviceScan::InclusiveSum(ctx->d_cub, cub_bytes, ctx->d_m_len, ctx->d_Mptr + 1, n,
+                                                 ctx->stream));
+        constexpr int kScatterCols = 256 / kScatterLanes;
+        hipLaunchKernelGGL(scatter_columns_kernel, dim3((n + kScatterCols - 1) / kScatterCols), dim3(256), 0,
+                           ctx->stream, n, cap, ctx->d_m_len, ctx->d_m_idx, ctx->d_m_val, ctx->d_Mptr, ctx->d_Mind,
+                           ctx->d_Mval, ctx->d_counter + 63);
+    }
     if (mixed)
         hipLaunchKernelGGL(count_status_kernel, dim3(std::min(256, (n + 255) / 256)), dim3(256), 0, ctx->stream, n,
                            ctx->d_status, COL_FALLBACK, ctx->d_counter + 62);
@@ -1474,7 +1609,9 @@ extern "C" int mspai_build(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* 
         stats->first_bin_ms = t_first;
         stats->nnz = last;
         stats->ncols = n;
-        if ((rc = read_chain_counts(ctx, (int)(mixed ? bins.size() : fbins.size()), mixed, stats))) return rc;
+        const int nb = given ? kStaticKinds + (int)bins.size() : (int)(mixed ? bins.size() : fbins.size());
+        if (first >= 0) ctx->h_counter[first] = ctx->h_counter[16 + first] = n;  // not through a queue
+        if ((rc = read_chain_counts(ctx, nb, mixed, stats))) return rc;
         stats->n_cache_hits = a.cache_slots > 0 ? ctx->h_counter[48] : 0;
     }
     return MSPAI_OK;
@@ -1518,7 +1655,9 @@ extern "C" int mspai_build_noalloc(mspai_ctx* ctx, const mspai_opts* opts, int* 
     const int needs = (qrup ? kNeedQrUpdate : 0) | (opts->precision == 1 && !qrup ? kNeedMixed : 0);
     const ScratchLayout G = generic_layout(ctx, cap, opts->maxnew, adaptive, needs);
     std::vector<Bin> bins, fbins;
-    if (opts->binning && !ctx->d_up_ptr) {  // an upper pattern runs unbinned
+    if (given_pattern_build(ctx, opts)) {
+        fbins = static_wide_bin(ctx, cap, G, needs & ~kNeedMixed);
+    } else if (opts->binning && !ctx->d_up_ptr) {  // an upper pattern runs unbinned
         int t = table_for(ctx, opts);
         bins = bin_layouts(ctx, cap, opts->maxnew, adaptive, G, kTables[t], needs);
         fbins = (needs & kNeedMixed) ? bin_layouts(ctx, cap, opts->maxnew, adaptive, G, kTables[t],
@@ -1645,13 +1784,8 @@ extern "C" int mspai_backward(mspai_ctx* ctx, const mspai_opts* opts, const doub
     if ((rc = check_shapes(ctx))) return rc;
     const int n = ctx->ncols;
     const int cap = ctx->cap;
-    const int needs = kNeedBackward | (opts->precision == 1 ? kNeedMixed : 0);
-    const ScratchLayout G = generic_layout(ctx, cap, 1, false, needs);
-    std::vector<Bin> bins;
-    if (opts->binning) {
-        int t = table_for(ctx, opts);
-        bins = bin_layouts(ctx, cap, 1, false, G, kTables[t], needs);
-    }
+    const ScratchLayout G = generic_layout(ctx, cap, 1, false, kNeedBackward);
+    const std::vector<Bin> wide = opts->binning ? static_wide_bin(ctx, cap, G, kNeedBackward) : std::vector<Bin>{};
     int gwaves = 0;
     if ((rc = prepare_generic(ctx, G, &gwaves))) return rc;
     HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
@@ -1665,9 +1799,13 @@ extern "C" int mspai_backward(mspai_ctx* ctx, const mspai_opts* opts, const doub
     a.gC = d_gC;
     a.gB = d_gB;
     a.cap = cap;
-    const bool mixed = opts->precision == 1 && !bins.empty();
     HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
-    if ((rc = run_chain(ctx, a, bins, bins, G, gwaves, mixed, 2, n))) return rc;
+    int first = -1;
+    if (opts->binning) {
+        if ((rc = run_static(ctx, a, wide, G, gwaves, 2, opts->precision == 1, n, cap, (double)ctx->nnzM / n, &first))) return rc;
+    } else {
+        if ((rc = run_chain(ctx, a, wide, wide, G, gwaves, false, 2, n))) return rc;
+    }
     HIPCHK(hipEventRecord(ctx->ev[2], ctx->stream));
     HIPCHK(hipEventRecord(ctx->ev[3], ctx->stream));
     if ((rc = fetch_counters(ctx))) return rc;
@@ -1684,7 +1822,8 @@ extern "C" int mspai_backward(mspai_ctx* ctx, const mspai_opts* opts, const doub
         stats->solve_ms = t_solve;
         stats->nnz = ctx->nnz;
         stats->ncols = n;
-        if ((rc = read_chain_counts(ctx, (int)bins.size(), mixed, stats))) return rc;
+        if (first >= 0) ctx->h_counter[first] = ctx->h_counter[16 + first] = n;  // not through a queue
+        if ((rc = read_chain_counts(ctx, opts->binning ? kStaticKinds + (int)wide.size() : 0, false, stats))) return rc;
     }
     return MSPAI_OK;
 }

@@ -101,6 +101,7 @@ struct BuildArgs {
     double epsilon;
     int maxnew, ns, use_mean;
     int cap;                // capacity of one output column
+    int direct;             // static build: column k's outputs at p_ptr[k] (M has the start pattern) instead of k*cap
     const int* queue;       // columns to build in this launch
     int nqueue;
     int* counter;           // persistent work-queue head

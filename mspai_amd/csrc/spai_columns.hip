@@ -112,6 +112,13 @@ __device__ __forceinline__ WaveScratch wave_scratch(char* ws, char* tie, const S
     return s;
 }
 
+/* First output slot of a column: its room of a.cap entries, or in a static
+ * build its place in the start pattern. */
+__device__ __forceinline__ size_t output_slot(const BuildArgs& a, int col)
+{
+    return a.direct ? (size_t)a.p_ptr[col] : (size_t)col * a.cap;
+}
+
 constexpr int kOverflow = -2;
 constexpr int kGenericHashSlots = 2048;  // LDS of the generic kernel's score hash (8 KB per wave)
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, 32 CUs each
@@ -715,44 +722,6 @@ __device__ __forceinline__ int refine_regs(const ScratchLayout& L, const WaveScr
     }
     if (lane < n) s.b[lane] = x;
     __syncthreads();
-    return kFallback;
-}
-
-/* The mixed adjoint's solve R^T R lambda = gbar with the FP32 register QR's
- * R, refined in FP64 as the forward solve is: rows of A(I,J) in registers,
- * u = A lambda per row, A^T u by reduce-scatter, lambda += (R^T R)^-1
- * (gbar - A^T u) until max|d| <= 1e-10 max|lambda|.  gbar in s.g on entry,
- * lambda there on return; kFallback when it does not converge. */
-template <int G, int NV>
-__device__ __forceinline__ int refine_adjoint_regs(const ScratchLayout& L, const WaveScratch& s, int m, int n)
-{
-    using Gr = Group<G>;
-    const int lane = Gr::lane();
-    const int ld = L.capI, ldq = L.ldq;
-    const float* q = s.aq32;
-    const bool row = lane < m;
-    double a[NV];
-#pragma unroll
-    for (int j = 0; j < NV; ++j) a[j] = (row && j < n) ? s.aqr[j * ld + lane] : 0.0;
-    const double dinv = lane < n ? 1.0 / (double)q[lane * ldq + lane] : 0.0;
-    const double gbar = lane < n ? s.g[lane] : 0.0;
-    double lam = normal_solve_lanes<G>(q, ldq, gbar, n, dinv);
-    for (int it = 0; it < kRefineSteps; ++it) {
-        double u = 0.0;  // (A lambda)_i on lane i
-#pragma unroll
-        for (int j = 0; j < NV; ++j)
-            if (j < n) u = __fma_rn(bcast_k<G>(lam, j), a[j], u);
-        const double h = rows_t_times<G, NV>(a, row ? u : 0.0, n);
-        const double d = normal_solve_lanes<G>(q, ldq, lane < n ? gbar - h : 0.0, n, dinv);
-        lam += d;
-        const double dmx = Gr::max(lane < n ? fabs(d) : 0.0);
-        const double lmx = Gr::max(lane < n ? fabs(lam) : 0.0);
-        if (dmx <= 1e-10 * lmx) {
-            if (lane < n) s.g[lane] = lam;
-            __syncthreads();
-            return 0;
-        }
-    }
     return kFallback;
 }
 
@@ -2133,7 +2102,9 @@ __device__ __forceinline__ void count_solve(const BuildArgs& a, const WaveScratc
     wk[7] += dn;
 }
 
-template <int G, bool kMixed, int NMAX, bool kHbm>
+/* The adjoint of one column of M (pattern in p_ptr/p_ind, values m_in) for
+ * columns wider than the given-pattern kernels take: |J| up to the layout's. */
+template <int G, bool kHbm>
 __device__ __forceinline__ int backward_column(const BuildArgs& a, const ScratchLayout& L, const WaveScratch& s,
                                                int col)
 {
@@ -2152,71 +2123,14 @@ __device__ __forceinline__ int backward_column(const BuildArgs& a, const Scratch
     int m = build_I<G, kHbm>(a, L, s, n);
     if (m == kOverflow) return kMoveOn;
     if (m < n) return kDone;  // degenerate column: no gradient
-    gather_ahat<G, kMixed && NMAX == 0>(a, L, s, m, n);
+    gather_ahat<G, false>(a, L, s, m, n);
     make_rhs<G>(a, s, m, col);
-    /* the register QRs leave A(I,J) intact in LDS: products from it */
-    const bool regs = NMAX > 0 && m <= G && n <= NMAX;
-    const double* R = s.aqr;
-    int ldr = ld;
-    if (kMixed) {
-        if (regs) {
-            if (qr_regs_f32<G, (NMAX > 0 ? NMAX : 4)>(L, s, m, n) == kFallback) return kRedoFp64;
-        } else if (NMAX > 0 || qr_f32<G>(L, s, m, n) == kFallback) {
-            return kRedoFp64;  // (register bins hold register columns only)
-        }
-    } else if (regs) {
-        int st2;
-        if constexpr (G == kWave && NMAX == 32)
-            st2 = ls_solve_rows64<true>(L, s, m, n);
-        else
-            st2 = ls_solve_regs<G, (NMAX > 0 ? NMAX : 4), true>(L, s, m, n);
-        if (st2 & (COL_SINGULAR | COL_UNDERDET)) return kDone;
-        R = s.rq;
-        ldr = L.capJ;
-    } else {
-        if (ls_solve<G>(L, s, m, n) & (COL_SINGULAR | COL_UNDERDET)) return kDone;
-    }
-    const bool dense = kMixed || regs;
+    if (ls_solve<G>(L, s, m, n) & (COL_SINGULAR | COL_UNDERDET)) return kDone;
     /* r = b - C m (into s.r) */
-    csc_apply<G>(a, L, s, m, n, s.y, s.b0, s.r, dense);
-    int rst = 1;  // 1: not refined in registers
-    if constexpr (kMixed && NMAX > 0) {
-        /* 16- and 64-lane groups, and 32-lane groups with |J| <= 8 */
-        if (regs && (G != 32 || n <= 8)) rst = refine_adjoint_regs<G, (G == 64 ? 32 : 8)>(L, s, m, n);
-        if (rst == kFallback) return kRedoFp64;
-    }
-    if (kMixed && rst != 0) {
-        for (int i = lane; i < n; i += G) s.z[i] = s.g[i];
-        __syncthreads();
-        normal_solve<G>(s.aq32, L.ldq, s.g, n);
-        bool ok = false;
-        for (int it = 0; it < kRefineSteps; ++it) {
-            csc_apply<G>(a, L, s, m, n, s.g, nullptr, s.b0, true);  // u = C lambda
-            csc_apply_t<G>(a, L, s, m, n, s.b0, s.b, true);          // C^T u
-            for (int i = lane; i < n; i += G) s.b[i] = s.z[i] - s.b[i];
-            __syncthreads();
-            normal_solve<G>(s.aq32, L.ldq, s.b, n);
-            double dmx = 0.0, lmx = 0.0;
-            for (int i = lane; i < n; i += G) {
-                double l = s.g[i] + s.b[i];
-                s.g[i] = l;
-                dmx = fmax(dmx, fabs(s.b[i]));
-                lmx = fmax(lmx, fabs(l));
-            }
-            dmx = Gr::max(dmx);
-            lmx = Gr::max(lmx);
-            __syncthreads();
-            if (dmx <= 1e-10 * lmx) {
-                ok = true;
-                break;
-            }
-        }
-        if (!ok) return kRedoFp64;
-    } else if (!kMixed) {
-        normal_solve<G>(R, ldr, s.g, n);
-    }
+    csc_apply<G>(a, L, s, m, n, s.y, s.b0, s.r, false);
+    normal_solve<G>(s.aqr, ld, s.g, n);
     /* s = C lambda (into s.b0) */
-    csc_apply<G>(a, L, s, m, n, s.g, nullptr, s.b0, dense);
+    csc_apply<G>(a, L, s, m, n, s.g, nullptr, s.b0, false);
     /* dL/dC_ij += r_i lambda_j - s_i m_j over the stored entries of J (the
      * column segments build_I left) */
     const int total = s.segoff[n];
@@ -2650,7 +2564,7 @@ __device__ __forceinline__ void save_column_state(const BuildArgs& a, const Wave
                                                   int st, const int (&near)[3], double wk, bool counters)
 {
     const int lane = Group<G>::lane();
-    const size_t o = (size_t)col * a.cap;
+    const size_t o = output_slot(a, col);
     if (!a.save_state) {
         if (lane == 0) a.nsolve[col] = 0;
         __syncthreads();
@@ -2679,7 +2593,7 @@ __device__ __forceinline__ int solve_column(const BuildArgs& a, const ScratchLay
     double* wk = a.work ? s.wsum : nullptr;  // summed in LDS, stored with the column
     int st = 0, step0 = -1, n;
     int near[3] = {0, 0, 0};  // near-margin decisions (counters builds, FP64)
-    const size_t o = (size_t)col * a.cap;
+    const size_t o = output_slot(a, col);
     const int mark = a.nsolve[col];
     const int* jsrc;
     if (mark < 0) {
@@ -2827,8 +2741,8 @@ __device__ __forceinline__ void wave_append(bool flag, int col, int* out, int* c
     if (flag) out[base + __popcll(mask & ((1ull << lane_id()) - 1ull))] = col;
 }
 
-/* kMode: 0 FP64 build, 1 mixed build, 2 FP64 adjoint, 3 mixed adjoint,
- * 4 FP64 build with the dense QR update (-qr 2).  The second launch bound is
+/* kMode: 0 FP64 build, 1 mixed build, 2 adjoint, 4 FP64 build with the dense
+ * QR update (-qr 2).  The second launch bound is
  * the resident waves per SIMD the register allocation must allow where LDS
  * would admit more than the registers otherwise do: 5 for the FP64 8-wide
  * 32-lane kernel, 4 for its other modes and the generic (HBM working set)
@@ -2912,15 +2826,15 @@ __global__ __launch_bounds__(64, kWaves > 0 ? kWaves
                 col = queue[q];
                 if (kMode < 2)
                     outcome = solve_column<G, kMode == 1, NMAX, !kLds, kWaves == 1>(a, L, s, col);
-                else if (kMode < 4)
-                    outcome = backward_column<G, kMode == 3, NMAX, !kLds>(a, L, s, col);
+                else if (kMode == 2)
+                    outcome = backward_column<G, !kLds>(a, L, s, col);
                 else
                     outcome = solve_column_qrup<G, !kLds>(a, L, s, col);
             }
             __syncthreads();
             const bool leader = Group<G>::lane() == 0;
             wave_append(leader && outcome == kMoveOn, col, a.overflow, a.n_overflow);
-            if (kMode == 1 || kMode == 3) wave_append(leader && outcome == kRedoFp64, col, a.fallback, a.n_fallback);
+            if (kMode == 1) wave_append(leader && outcome == kRedoFp64, col, a.fallback, a.n_fallback);
         }
     }
 }
@@ -3086,18 +3000,7 @@ static ColumnKernel binned_kernel(const ScratchLayout& L, int group, int mode, i
          * 2 waves per SIMD, where LDS would hold 11 per CU) */
         if (regs && L.capJ <= 16) return &spai_column_kernel<64, true, 1, 16, 3>;
         return regs ? &spai_column_kernel<64, true, 1, 32> : &spai_column_kernel<64, true, 1, 0>;
-    case 2:
-        if (group == 16) return regs ? &spai_column_kernel<16, true, 2, 8> : &spai_column_kernel<16, true, 2, 0>;
-        if (group == 32)
-            return regs ? (L.capJ <= 8 ? &spai_column_kernel<32, true, 2, 8> : &spai_column_kernel<32, true, 2, 16>)
-                        : &spai_column_kernel<32, true, 2, 0>;
-        return regs ? &spai_column_kernel<64, true, 2, 32> : &spai_column_kernel<64, true, 2, 0>;
-    case 3:
-        if (group == 16) return regs ? &spai_column_kernel<16, true, 3, 8> : &spai_column_kernel<16, true, 3, 0>;
-        if (group == 32)
-            return regs ? (L.capJ <= 8 ? &spai_column_kernel<32, true, 3, 8> : &spai_column_kernel<32, true, 3, 16>)
-                        : &spai_column_kernel<32, true, 3, 0>;
-        return regs ? &spai_column_kernel<64, true, 3, 32> : &spai_column_kernel<64, true, 3, 0>;
+    case 2: return &spai_column_kernel<64, true, 2, 0>;  // the given-pattern kernels' overflow
     default: MSPAI_PICK(4);
     }
 #undef MSPAI_PICK

@@ -38,6 +38,20 @@ void launch_copy_ints(const int* src, int* dst, int count, hipStream_t stream);
 void launch_fp64_generic(const BuildArgs& a, const ScratchLayout& L, int mode, const int* queue,
                          const int* nqueue, int* head, int nwaves, hipStream_t stream);
 
+/* Column kernels for a given pattern (spai_static.hip): static FP64 build, or
+ * with `back` the adjoint.  Kind k takes columns of |J| <= kStaticJ[k] and
+ * |I| <= kStaticI[k]: those of queue (length *nqueue), or without a queue all
+ * columns 0..nall; others go to a.overflow.  The build writes m_val at the
+ * start pattern's places (a.direct). */
+constexpr int kStaticKinds = 3;
+constexpr int kStaticJ[kStaticKinds] = {7, 15, 31};
+constexpr int kStaticI[kStaticKinds] = {32, 64, 64};
+void launch_static_columns(int kind, const BuildArgs& a, bool back, bool refine, const int* queue, const int* nqueue, int nall,
+                           int num_cu, hipStream_t stream);
+/* colptr, rowind and *count (entries) of an M that has the start pattern. */
+void launch_copy_pattern(int ncols, int nnz, const int* p_ptr, const int* p_ind, int* colptr, int* rowind,
+                         int* count, hipStream_t stream);
+
 /* Sparse products (apply.hip). */
 void launch_fill_int(int* p, long long count, int value, hipStream_t stream);
 /* col_of[e] = column of CSC entry e, order[e] = e. */
