@@ -90,19 +90,7 @@ __global__ __launch_bounds__(kLineBlock) void line_dot_kernel(int nlines, const 
     if (i < nlines) y[i] = sum;
 }
 
-__global__ void fill_int_kernel(int* p, long long count, int value)
-{
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count) p[i] = value;
-}
-
 }  // namespace
-
-void launch_fill_int(int* p, long long count, int value, hipStream_t stream)
-{
-    if (count <= 0) return;
-    hipLaunchKernelGGL(fill_int_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream, p, count, value);
-}
 
 void launch_csr_entry_cols(const int* colptr, int ncols, int* col_of, int* order, hipStream_t stream)
 {

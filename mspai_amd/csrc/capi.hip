@@ -27,6 +27,15 @@ using namespace mspai;
 
 constexpr int kMaxBins = 4;
 constexpr int kMaxLaunch = 2 * kMaxBins + 2;  // column-kernel launches of one build: mixed bins, FP64 bins, generic
+/* Time stamps of a build, written by the kernels themselves as they start (an
+ * event between two launches holds the stream for several microseconds): one
+ * per column-kernel launch, then these.  A launch ends where the next
+ * begins. */
+constexpr int kStampStart = kMaxLaunch;         // counters cleared
+constexpr int kStampRoute = kMaxLaunch + 1;     // the routing kernel
+constexpr int kStampSolved = kMaxLaunch + 2;    // the column kernels done
+constexpr int kStampEnd = kMaxLaunch + 3;
+constexpr int kNumStamps = kMaxLaunch + 4;
 
 /* Device scratch of mspai_build_noalloc (queues, counters, output slots,
  * per-column results, tie buffers, the scan workspace and the generic
@@ -51,25 +60,34 @@ void dfree(T*& p)
     p = nullptr;
 }
 
-__global__ void column_norms_kernel(DevCsc A, double* ajn)
-{
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= A.ncols) return;
-    double s = 0.0;
-    for (int e = A.colptr[j]; e < A.colptr[j + 1]; ++e) {
-        double v = A.val[e];
-        s = __dadd_rn(s, __dmul_rn(v, v));
-    }
-    ajn[j] = sqrt(s);
-}
+/* Once per set of values, for the candidate scores, in one launch: blocks
+ * b < norm_blocks compute ||a_j|| of 256 columns (Euclidean_Norm: sequential,
+ * unfused, one column per thread); the others put C's values in the order of
+ * its row pattern (which holds exactly C's entries, sorted per row; rp_val
+ * nullptr: not wanted), kValueLanes lanes per column.  Every stored entry
+ * finds its column in its row by a binary search, a chain of dependent reads:
+ * latency-bound, so the lanes of a column search together -- 3.1 M entries in
+ * rows of 12: 200 us with one thread per column, 33 us so. */
+constexpr int kValueLanes = 8;
 
-/* C's values in the order of its row pattern (which holds exactly C's
- * entries, sorted per row): each stored entry finds its column in its row. */
-__global__ void row_values_kernel(DevCsc A, const int* rp_ptr, const int* rp_ind, double* rp_val)
+__global__ __launch_bounds__(256) void column_values_kernel(DevCsc A, double* ajn, int norm_blocks, const int* rp_ptr,
+                                                           const int* rp_ind, double* rp_val)
 {
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if ((int)blockIdx.x < norm_blocks) {
+        const int j = blockIdx.x * 256 + threadIdx.x;
+        if (j >= A.ncols) return;
+        double s = 0.0;
+        for (int e = A.colptr[j]; e < A.colptr[j + 1]; ++e) {
+            double v = A.val[e];
+            s = __dadd_rn(s, __dmul_rn(v, v));
+        }
+        ajn[j] = sqrt(s);
+        return;
+    }
+    const int j = ((int)blockIdx.x - norm_blocks) * (256 / kValueLanes) + (int)threadIdx.x / kValueLanes;
     if (j >= A.ncols) return;
-    for (int e = A.colptr[j]; e < A.colptr[j + 1]; ++e) {
+    const int end = A.colptr[j + 1];
+    for (int e = A.colptr[j] + (int)threadIdx.x % kValueLanes; e < end; e += kValueLanes) {
         const int i = A.rowind[e];
         int lo = rp_ptr[i], hi = rp_ptr[i + 1];
         while (lo < hi) {
@@ -98,45 +116,92 @@ __global__ void work_sum_kernel(const double* work, int n, double* out)
 }
 
 
-/* M's CSC from the per-column outputs: colptr[1..ncols] holds the inclusive
- * scan of the lengths; this kernel also sets colptr[0] = 0 and *nnz, and
- * counts the columns the FP64 kernels built in a mixed build (*nfp64). */
-/* Output slots -> CSC: kScatterLanes lanes per column (most columns hold
- * fewer entries), colptr from the scan of the lengths. */
-constexpr int kScatterLanes = 16;
+/* Compaction of the output slots into M's CSC in two launches of the same
+ * tiles of kTileCols columns: the entries of every tile (and the columns
+ * whose status has `bit`, when status is given), then, per tile, the sum of
+ * the tiles before it, the scan of its lengths and the copy of its entries,
+ * one thread per entry in CSC order (the column by a binary search of the
+ * tile's scan), so that the stores are contiguous. */
+constexpr int kTileCols = 256;
 
-__global__ void scatter_columns_kernel(int ncols, int cap, const int* m_len, const int* m_idx,
-                                       const double* m_val, int* colptr, int* rowind, double* val, int* nnz)
+__device__ __forceinline__ int block_sum(int v, int* part)
 {
-    const int col = blockIdx.x * (blockDim.x / kScatterLanes) + (int)(threadIdx.x / kScatterLanes);
-    const int sub = threadIdx.x % kScatterLanes;
-    if (col >= ncols) return;
-    const int len = m_len[col], o = col == 0 ? 0 : colptr[col];
-    if (sub == 0 && col == 0) colptr[0] = 0;
-    if (sub == 0 && col == ncols - 1) *nnz = o + len;
-    const size_t src = (size_t)col * cap;
-    for (int i = sub; i < len; i += kScatterLanes) {
-        rowind[o + i] = m_idx[src + i];
-        val[o + i] = m_val[src + i];
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+    __syncthreads();  // part's readers of a previous call are done
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return part[0] + part[1] + part[2] + part[3];
+}
+
+__global__ __launch_bounds__(kTileCols) void tile_sums_kernel(int ncols, const int* m_len, const int* status, int bit,
+                                                              int* tile_sum, int* nbit, unsigned long long* stamp)
+{
+    __shared__ int part[kTileCols / 64];
+    if (blockIdx.x == 0 && threadIdx.x == 0) *stamp = wall_clock64();
+    const int col = blockIdx.x * kTileCols + threadIdx.x;
+    const int sum = block_sum(col < ncols ? m_len[col] : 0, part);
+    if (threadIdx.x == 0) tile_sum[blockIdx.x] = sum;
+    if (status) {
+        const int c = block_sum(col < ncols && (status[col] & bit), part);
+        if (threadIdx.x == 0 && c) atomicAdd(nbit, c);
     }
 }
 
-/* *out += the columns whose status has `bit`: a grid-stride count, one
- * atomic per block (a per-column atomic on one address serializes). */
-__global__ __launch_bounds__(256) void count_status_kernel(int n, const int* status, int bit, int* out)
+__global__ __launch_bounds__(kTileCols) void compact_columns_kernel(int ncols, int cap, const int* m_len,
+                                                                    const int* m_idx, const double* m_val,
+                                                                    const int* tile_sum, int* colptr, int* rowind,
+                                                                    double* val, int* nnz)
 {
-    __shared__ int part[256 / 64];
-    int c = 0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        c += (status[i] & bit) != 0;
-    for (int off = 32; off > 0; off >>= 1) c += __shfl_down(c, off, 64);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = c;
+    __shared__ int part[kTileCols / 64];
+    __shared__ int first[kTileCols + 1];  // a column's first entry in the tile
+    const int t = threadIdx.x, c0 = blockIdx.x * kTileCols, col = c0 + t;
+    int before = 0;
+    for (int b = t; b < (int)blockIdx.x; b += kTileCols) before += tile_sum[b];
+    before = block_sum(before, part);
+    const int len = col < ncols ? m_len[col] : 0;
+    int incl = Group<64>::scan_incl(len);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int t = 0;
-        for (int w = 0; w < 256 / 64; ++w) t += part[w];
-        if (t) atomicAdd(out, t);
+    if ((t & 63) == 63) part[t >> 6] = incl;
+    __syncthreads();
+    for (int w = 0; w < (t >> 6); ++w) incl += part[w];
+    first[t + 1] = incl;
+    if (t == 0) first[0] = 0;
+    __syncthreads();
+    if (col < ncols) colptr[col + 1] = before + incl;
+    if (blockIdx.x == 0 && t == 0) colptr[0] = 0;
+    if (col == ncols - 1) *nnz = before + incl;
+    const int total = first[kTileCols];
+    for (int e = t; e < total; e += kTileCols) {
+        int lo = 0, hi = kTileCols - 1;  // the last column that starts at or before e
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (first[mid] <= e) lo = mid;
+            else hi = mid - 1;
+        }
+        const size_t src = (size_t)(c0 + lo) * cap + (e - first[lo]);
+        rowind[before + e] = m_idx[src];
+        val[before + e] = m_val[src];
     }
+}
+
+/* Start of a build or adjoint on the stream: the counters cleared (a kernel,
+ * not a memset node) and the start time. */
+__global__ void start_kernel(int* counter, unsigned long long* stamp)
+{
+    counter[threadIdx.x] = 0;
+    if (threadIdx.x == 0) *stamp = wall_clock64();
+}
+
+/* Nothing but a time stamp. */
+__global__ void stamp_kernel(unsigned long long* stamp) { *stamp = wall_clock64(); }
+
+/* End of one: counters and time stamps to the pinned host arrays. */
+__global__ void publish_kernel(const int* counter, int* h_counter, const unsigned long long* ts,
+                               unsigned long long* h_ts)
+{
+    const int t = threadIdx.x;
+    h_counter[t] = counter[t];
+    if (t < kNumStamps) h_ts[t] = t == kStampEnd ? wall_clock64() : ts[t];
 }
 
 }  // namespace
@@ -204,11 +269,14 @@ struct mspai_ctx {
     long long csr_tmp_cap = 0;
     bool a_csr_ok = false, m_csr_ok = false;
     bool ajn_ok = false;  // d_ajn (and d_rp_val) hold the column norms (row values) of the current values
-    hipEvent_t ev[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};  // [4..5]: first size bin
+    hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};  // block builds
     hipEvent_t csr_ev = nullptr;  // orders a CSR copy on the context's stream with the caller's stream
-    /* per-launch profile of the last build: events around every column-kernel
-     * launch, and (builds with counters) the totals of the columns each finished */
-    hipEvent_t lev[2 * kMaxLaunch] = {};
+    /* per-launch profile of the last build: time stamps (kStamp*; the device
+     * array and its pinned copy), and (builds with counters) the totals of
+     * the columns each launch finished */
+    unsigned long long *d_ts = nullptr, *h_ts = nullptr;
+    double ticks_per_ms = 1e5;
+    bool was_routed = false;  // the last build ran the routing kernel
     int nlaunch = 0;
     char lname[kMaxLaunch][48] = {};
     double* d_lwork = nullptr;  // kMaxLaunch x kLaunchStat
@@ -350,11 +418,9 @@ extern "C" int mspai_ctx_create(int device, mspai_ctx** out)
             delete ctx;
             return MSPAI_ERR_HIP;
         }
-    for (auto& e : ctx->lev)
-        if (hipEventCreate(&e) != hipSuccess) {
-            delete ctx;
-            return MSPAI_ERR_HIP;
-        }
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && khz > 0)
+        ctx->ticks_per_ms = khz;
     if (hipEventCreateWithFlags(&ctx->csr_ev, hipEventDisableTiming) != hipSuccess) {
         delete ctx;
         return MSPAI_ERR_HIP;
@@ -373,6 +439,9 @@ extern "C" int mspai_ctx_create(int device, mspai_ctx** out)
     }
     if (hipMalloc((void**)&ctx->d_counter, 64 * sizeof(int)) != hipSuccess ||
         hipHostMalloc((void**)&ctx->h_counter, 64 * sizeof(int), hipHostMallocDefault) != hipSuccess ||
+        hipMalloc((void**)&ctx->d_ts, kNumStamps * sizeof(unsigned long long)) != hipSuccess ||
+        hipHostMalloc((void**)&ctx->h_ts, kNumStamps * sizeof(unsigned long long), hipHostMallocDefault) !=
+            hipSuccess ||
         hipMalloc((void**)&ctx->d_wsum, kNumWork * sizeof(double)) != hipSuccess ||
         hipMalloc((void**)&ctx->d_lwork, kMaxLaunch * kLaunchStat * sizeof(double)) != hipSuccess) {
         delete ctx;
@@ -435,8 +504,8 @@ extern "C" int mspai_ctx_destroy(mspai_ctx* ctx)
     block_free(ctx);
     for (auto& e : ctx->ev)
         if (e) (void)hipEventDestroy(e);
-    for (auto& e : ctx->lev)
-        if (e) (void)hipEventDestroy(e);
+    dfree(ctx->d_ts);
+    if (ctx->h_ts) (void)hipHostFree(ctx->h_ts);
     if (ctx->csr_ev) (void)hipEventDestroy(ctx->csr_ev);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -1094,9 +1163,8 @@ static int waves_per_cu(const Bin& b, int mode)
     return w;
 }
 
-/* Per-launch profile: an event before and after each column-kernel launch,
- * the launch's name, and its slot of the counter totals (builds with
- * counters only; a.work is set exactly then). */
+/* Per-launch profile: the launch's time stamp and name, and its slot of the
+ * counter totals (builds with counters only; a.work is set exactly then). */
 static int begin_launch(mspai_ctx* ctx, BuildArgs& a, const char* what, int mode, int bin, const Bin* b)
 {
     const int k = ctx->nlaunch;
@@ -1108,15 +1176,38 @@ static int begin_launch(mspai_ctx* ctx, BuildArgs& a, const char* what, int mode
     else
         std::snprintf(ctx->lname[k], sizeof ctx->lname[k], "%s %s", kModes[mode], what);
     a.lwork = a.work ? ctx->d_lwork + (size_t)k * kLaunchStat : nullptr;
-    HIPCHK(hipEventRecord(ctx->lev[2 * k], ctx->stream));
+    a.stamp = ctx->d_ts + k;
+    ctx->nlaunch++;
     return MSPAI_OK;
 }
 
-static int end_launch(mspai_ctx* ctx)
+/* Start of a build or adjoint: counters cleared, no launches yet. */
+static int start_build(mspai_ctx* ctx)
 {
-    HIPCHK(hipEventRecord(ctx->lev[2 * ctx->nlaunch + 1], ctx->stream));
-    ctx->nlaunch++;
+    hipLaunchKernelGGL(start_kernel, dim3(1), dim3(64), 0, ctx->stream, ctx->d_counter, ctx->d_ts + kStampStart);
+    HIPCHK(hipGetLastError());
+    ctx->nlaunch = 0;
+    ctx->was_routed = false;
     return MSPAI_OK;
+}
+
+static double stamp_ms(const mspai_ctx* ctx, int from, int to)
+{
+    return (double)(ctx->h_ts[to] - ctx->h_ts[from]) / ctx->ticks_per_ms;
+}
+
+/* Duration of column-kernel launch k of the last build. */
+static double launch_ms(const mspai_ctx* ctx, int k)
+{
+    return stamp_ms(ctx, k, k + 1 < ctx->nlaunch ? k + 1 : kStampSolved);
+}
+
+/* Times of the last build into stats (the stream is synchronized). */
+static void build_times(const mspai_ctx* ctx, mspai_stats* stats)
+{
+    stats->build_ms = stamp_ms(ctx, kStampStart, kStampEnd);
+    stats->solve_ms = ctx->nlaunch > 0 ? stamp_ms(ctx, ctx->was_routed ? kStampRoute : 0, kStampSolved) : 0.0;
+    stats->first_bin_ms = ctx->nlaunch > 0 ? launch_ms(ctx, 0) : 0.0;
 }
 
 /* HBM tie-path buffers of the LDS bins: one region per resident group (the
@@ -1149,7 +1240,7 @@ constexpr int kDirectFp64 = 4096;
  * [8..16) heads, [16..24) routed lengths, mixed [24..32) lengths, [32..40)
  * heads, [40] blocks of the routing kernel done. */
 static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins, const std::vector<Bin>& fbins,
-                     const ScratchLayout& G, int gwaves, bool mixed, int fp64_mode, int n)
+                     const ScratchLayout& G, int gwaves, bool mixed, int fp64_mode, int n, int longest)
 {
     const int nb = (int)bins.size();
     const int nf = (int)fbins.size();
@@ -1160,6 +1251,15 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
         edges.capSort[b] = routed[b].L.capSid;  // the I-set raw list of the start pattern
         edges.capI[b] = routed[b].L.capI;
     }
+    /* when no start pattern can outgrow the first bin (|J0| at most `longest`,
+     * rows at most their entries), the bin takes all columns by index and the
+     * routing kernel is not run (70 us of 0.26 million columns, 22 us of 65
+     * thousand) */
+    const size_t raw = (size_t)longest * ctx->maxcolnnz;
+    const bool straight = fp64_mode == 0 && !routed.empty() && longest <= routed[0].L.capJ &&
+                          raw <= (size_t)std::min(routed[0].L.capI, routed[0].L.capSid);
+    ctx->was_routed = !straight;
+    a.nqueue = n;
     int* counts = ctx->d_counter;
     int* heads = ctx->d_counter + 8;
     int* mcounts = ctx->d_counter + 24;
@@ -1167,9 +1267,6 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
     int* fq = ctx->d_queues;
     int* mq = ctx->d_queues + (size_t)(kMaxBins + 1) * n;
     int rc;
-    launch_fill_int(ctx->d_counter, 64, 0, ctx->stream);  // a kernel, not a memset node
-    HIPCHK(hipGetLastError());
-    ctx->nlaunch = 0;
     ctx->lwork_valid = a.work != nullptr;
     if (a.work) HIPCHK(hipMemsetAsync(ctx->d_lwork, 0, kMaxLaunch * kLaunchStat * sizeof(double), ctx->stream));
     a.status_or = 0;
@@ -1198,8 +1295,10 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
         const bool direct = fp64_mode == 0 && skip == nf && ctx->mixed_fp64_last >= 0 &&
                             ctx->mixed_fp64_last <= kDirectFp64 && !Lm.gram;
         const int to = direct ? 0 : skip;  // FP64 queue of the mixed chain's overflow
-        launch_classify(a, nb, edges, mq, mcounts, fq, counts, n, ctx->d_counter + 40, ctx->d_counter + 16,
-                        ctx->stream);
+        a.stamp = ctx->d_ts + kStampRoute;
+        if (!straight)
+            launch_classify(a, nb, edges, mq, mcounts, fq, counts, n, ctx->d_counter + 40, ctx->d_counter + 16,
+                            ctx->stream);
         HIPCHK(hipGetLastError());
         a.fallback = fq;
         a.n_fallback = counts;
@@ -1215,13 +1314,10 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
             const int mode = bins[b].fp64 ? fp64_mode : 1;
             int per_cu = waves_per_cu(bins[b], mode);
             const ScratchLayout& L = bins[b].L;
-            if (b == 0) HIPCHK(hipEventRecord(ctx->ev[4], ctx->stream));
             if ((rc = begin_launch(ctx, a, nullptr, mode, b, &bins[b]))) return rc;
-            launch_binned(a, L, grp, mode, mq + (size_t)b * n, mcounts + b, mheads + b, ctx->num_cu * per_cu,
+            launch_binned(a, L, grp, mode, straight && b == 0 ? nullptr : mq + (size_t)b * n, mcounts + b, mheads + b, ctx->num_cu * per_cu,
                           ctx->stream, bins[b].wcap);
             HIPCHK(hipGetLastError());
-            if ((rc = end_launch(ctx))) return rc;
-            if (b == 0) HIPCHK(hipEventRecord(ctx->ev[5], ctx->stream));
         }
         a.status_or = COL_FALLBACK;
         a.save_state = 0;
@@ -1233,11 +1329,13 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
             if ((rc = begin_launch(ctx, a, "generic (HBM working set)", fp64_mode, -1, nullptr))) return rc;
             launch_fp64_generic(a, G, fp64_mode, fq, counts, heads + nf, gwaves, ctx->stream);
             HIPCHK(hipGetLastError());
-            return end_launch(ctx);
+            return MSPAI_OK;
         }
     } else {
-        launch_classify(a, nf, edges, fq, counts, fq + (size_t)nf * n, counts + nf, n, ctx->d_counter + 40,
-                        ctx->d_counter + 16, ctx->stream);
+        a.stamp = ctx->d_ts + kStampRoute;
+        if (!straight)
+            launch_classify(a, nf, edges, fq, counts, fq + (size_t)nf * n, counts + nf, n, ctx->d_counter + 40,
+                            ctx->d_counter + 16, ctx->stream);
         HIPCHK(hipGetLastError());
     }
     a.fallback = nullptr;
@@ -1248,25 +1346,19 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
         a.n_overflow = counts + b + 1;
         int per_cu = waves_per_cu(fbins[b], fp64_mode);
         const ScratchLayout& L = fbins[b].L;
-        const bool first = b == 0 && !mixed;
         a.save_state = fp64_mode == 0;  // FP64 builds resume in the next bin (not the QR update or the adjoint)
-        if (first) HIPCHK(hipEventRecord(ctx->ev[4], ctx->stream));
         if ((rc = begin_launch(ctx, a, nullptr, fp64_mode, b, &fbins[b]))) return rc;
-        launch_binned(a, L, grp, fp64_mode, fq + (size_t)b * n, counts + b, heads + b,
+        launch_binned(a, L, grp, fp64_mode, straight && !mixed && b == 0 ? nullptr : fq + (size_t)b * n, counts + b,
+                      heads + b,
                       ctx->num_cu * per_cu, ctx->stream, fbins[b].wcap);
         HIPCHK(hipGetLastError());
-        if ((rc = end_launch(ctx))) return rc;
-        if (first) HIPCHK(hipEventRecord(ctx->ev[5], ctx->stream));
     }
     a.overflow = fq;  // never written: the generic layout holds every column
     a.n_overflow = counts + 7;
     a.save_state = 0;
-    if (nf == 0) HIPCHK(hipEventRecord(ctx->ev[4], ctx->stream));  // no bins: the generic kernel is the first
     if ((rc = begin_launch(ctx, a, "generic (HBM working set)", fp64_mode, -1, nullptr))) return rc;
     launch_fp64_generic(a, G, fp64_mode, fq + (size_t)nf * n, counts + nf, heads + nf, gwaves, ctx->stream);
     HIPCHK(hipGetLastError());
-    if ((rc = end_launch(ctx))) return rc;
-    if (nf == 0) HIPCHK(hipEventRecord(ctx->ev[5], ctx->stream));
     return MSPAI_OK;
 }
 
@@ -1298,9 +1390,6 @@ static int run_static(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& wide
     int* heads = ctx->d_counter + 8;
     int* q = ctx->d_queues;
     int rc;
-    launch_fill_int(ctx->d_counter, 64, 0, ctx->stream);  // a kernel, not a memset node
-    HIPCHK(hipGetLastError());
-    ctx->nlaunch = 0;
     ctx->lwork_valid = false;
     a.status_or = 0;
     a.save_state = 0;
@@ -1327,11 +1416,12 @@ static int run_static(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& wide
             edges.capI[kStaticKinds] = b.L.capI;
             edges.capSort[kStaticKinds] = b.L.capSid;
         }
+        ctx->was_routed = true;
+        a.stamp = ctx->d_ts + kStampRoute;
         launch_classify(a, nf, edges, q, counts, q + (size_t)nf * n, counts + nf, n, ctx->d_counter + 40,
                         ctx->d_counter + 16, ctx->stream);
         HIPCHK(hipGetLastError());
     }
-    HIPCHK(hipEventRecord(ctx->ev[4], ctx->stream));
     bool all_fit = false;
     for (int b = std::max(*first, 0); b < kStaticKinds && !all_fit; ++b) {
         /* past the kind that takes every column, only one with room for more rows */
@@ -1348,8 +1438,6 @@ static int run_static(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& wide
         launch_static_columns(b, a, back, refine, direct ? nullptr : q + (size_t)b * n, counts + b, n, ctx->num_cu,
                               ctx->stream);
         HIPCHK(hipGetLastError());
-        if ((rc = end_launch(ctx))) return rc;
-        if (b == std::max(*first, 0)) HIPCHK(hipEventRecord(ctx->ev[5], ctx->stream));
         /* no column of the pattern can have more rows than this kind takes */
         all_fit = direct && (size_t)longest * ctx->maxcolnnz <= (size_t)kStaticI[b];
     }
@@ -1362,21 +1450,22 @@ static int run_static(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& wide
         launch_binned(a, wide[b].L, wide[b].group, mode, q + (size_t)t * n, counts + t, heads + t,
                       ctx->num_cu * waves_per_cu(wide[b], mode), ctx->stream, wide[b].wcap);
         HIPCHK(hipGetLastError());
-        if ((rc = end_launch(ctx))) return rc;
     }
     a.overflow = q;  // never written: the generic layout holds every column
     a.n_overflow = counts + 7;
     if ((rc = begin_launch(ctx, a, "generic (HBM working set)", mode, -1, nullptr))) return rc;
     launch_fp64_generic(a, G, mode, q + (size_t)nf * n, counts + nf, heads + nf, gwaves, ctx->stream);
     HIPCHK(hipGetLastError());
-    return end_launch(ctx);
+    return MSPAI_OK;
 }
 
-/* Queue the copy of the counters to the pinned host array (after the last
- * kernel of a build on the stream; read once the stream is synchronized). */
+/* Counters and time stamps to the pinned host arrays (after the last kernel
+ * of a build on the stream; read once the stream is synchronized). */
 static int fetch_counters(mspai_ctx* ctx)
 {
-    HIPCHK(hipMemcpyAsync(ctx->h_counter, ctx->d_counter, 64 * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+    hipLaunchKernelGGL(publish_kernel, dim3(1), dim3(64), 0, ctx->stream, ctx->d_counter, ctx->h_counter, ctx->d_ts,
+                       ctx->h_ts);
+    HIPCHK(hipGetLastError());
     return MSPAI_OK;
 }
 
@@ -1512,13 +1601,12 @@ extern "C" int mspai_build(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* 
     int gwaves = 0;
     if ((rc = prepare_generic(ctx, G, &gwaves))) return rc;
 
-    HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
+    if ((rc = start_build(ctx))) return rc;
     BuildArgs a = base_args(ctx);
     if (adaptive && !ctx->ajn_ok) {  // once per set of values; only the candidate scores read them
-        hipLaunchKernelGGL(column_norms_kernel, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, a.A, ctx->d_ajn);
-        if (a.rp_val)
-            hipLaunchKernelGGL(row_values_kernel, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, a.A, a.rp_ptr,
-                               a.rp_ind, ctx->d_rp_val);
+        const int nblk = (n + 255) / 256, vblk = a.rp_val ? (n + 256 / kValueLanes - 1) / (256 / kValueLanes) : 0;
+        hipLaunchKernelGGL(column_values_kernel, dim3(nblk + vblk), dim3(256), 0, ctx->stream, a.A, ctx->d_ajn, nblk,
+                           a.rp_ptr, a.rp_ind, ctx->d_rp_val);
         HIPCHK(hipGetLastError());
         ctx->ajn_ok = true;
     }
@@ -1559,33 +1647,28 @@ extern "C" int mspai_build(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* 
         a.cache_data = ctx->d_cache_data;
         a.cache_hits = ctx->d_counter + 48;
     }
-    HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
     int first = -1;
     if (given) {
         if ((rc = run_static(ctx, a, bins, G, gwaves, 0, opts->precision == 1, n, ctx->plen_max, (double)ctx->p_nnz / n, &first))) return rc;
     } else {
-        if ((rc = run_chain(ctx, a, bins, fbins, G, gwaves, mixed, qrup ? 4 : 0, n))) return rc;
+        if ((rc = run_chain(ctx, a, bins, fbins, G, gwaves, mixed, qrup ? 4 : 0, n,
+                            ctx->plen_max)))
+            return rc;
     }
-    HIPCHK(hipEventRecord(ctx->ev[2], ctx->stream));
-
+    unsigned long long* const solved = ctx->d_ts + kStampSolved;
     if (given) {
         launch_copy_pattern(n, ctx->p_nnz, ctx->d_p_ptr, ctx->d_p_ind, ctx->d_Mptr, ctx->d_Mind,
-                            ctx->d_counter + 63, ctx->stream);
+                            ctx->d_counter + 63, solved, ctx->stream);
     } else {
-        /* compaction: colptr[0] = 0, colptr[1..n] = inclusive scan of the lengths */
-        size_t cub_bytes = ctx->cub_bytes;
-        HIPCHK(hipcub::DeviceScan::InclusiveSum(ctx->d_cub, cub_bytes, ctx->d_m_len, ctx->d_Mptr + 1, n,
-                                                 ctx->stream));
-        constexpr int kScatterCols = 256 / kScatterLanes;
-        hipLaunchKernelGGL(scatter_columns_kernel, dim3((n + kScatterCols - 1) / kScatterCols), dim3(256), 0,
-                           ctx->stream, n, cap, ctx->d_m_len, ctx->d_m_idx, ctx->d_m_val, ctx->d_Mptr, ctx->d_Mind,
+        /* the queues are empty now: the tiles' sums go there */
+        const int tiles = (n + kTileCols - 1) / kTileCols;
+        hipLaunchKernelGGL(tile_sums_kernel, dim3(tiles), dim3(kTileCols), 0, ctx->stream, n, ctx->d_m_len,
+                           mixed ? ctx->d_status : nullptr, COL_FALLBACK, ctx->d_queues, ctx->d_counter + 62, solved);
+        hipLaunchKernelGGL(compact_columns_kernel, dim3(tiles), dim3(kTileCols), 0, ctx->stream, n, cap,
+                           ctx->d_m_len, ctx->d_m_idx, ctx->d_m_val, ctx->d_queues, ctx->d_Mptr, ctx->d_Mind,
                            ctx->d_Mval, ctx->d_counter + 63);
     }
-    if (mixed)
-        hipLaunchKernelGGL(count_status_kernel, dim3(std::min(256, (n + 255) / 256)), dim3(256), 0, ctx->stream, n,
-                           ctx->d_status, COL_FALLBACK, ctx->d_counter + 62);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipEventRecord(ctx->ev[3], ctx->stream));
     if ((rc = fetch_counters(ctx))) return rc;
     HIPCHK(hipStreamSynchronize(ctx->stream));
 
@@ -1599,18 +1682,12 @@ extern "C" int mspai_build(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* 
     ctx->last_counters = opts->counters != 0;
     if (stats) {
         std::memset(stats, 0, sizeof(*stats));
-        float t_all = 0, t_solve = 0;
-        HIPCHK(hipEventElapsedTime(&t_all, ctx->ev[0], ctx->ev[3]));
-        HIPCHK(hipEventElapsedTime(&t_solve, ctx->ev[1], ctx->ev[2]));
-        stats->build_ms = t_all;
-        stats->solve_ms = t_solve;
-        float t_first = 0;
-        HIPCHK(hipEventElapsedTime(&t_first, ctx->ev[4], ctx->ev[5]));
-        stats->first_bin_ms = t_first;
+        build_times(ctx, stats);
         stats->nnz = last;
         stats->ncols = n;
         const int nb = given ? kStaticKinds + (int)bins.size() : (int)(mixed ? bins.size() : fbins.size());
         if (first >= 0) ctx->h_counter[first] = ctx->h_counter[16 + first] = n;  // not through a queue
+        if (!given && !ctx->was_routed) ctx->h_counter[mixed ? 24 : 0] = ctx->h_counter[16] = n;
         if ((rc = read_chain_counts(ctx, nb, mixed, stats))) return rc;
         stats->n_cache_hits = a.cache_slots > 0 ? ctx->h_counter[48] : 0;
     }
@@ -1788,7 +1865,7 @@ extern "C" int mspai_backward(mspai_ctx* ctx, const mspai_opts* opts, const doub
     const std::vector<Bin> wide = opts->binning ? static_wide_bin(ctx, cap, G, kNeedBackward) : std::vector<Bin>{};
     int gwaves = 0;
     if ((rc = prepare_generic(ctx, G, &gwaves))) return rc;
-    HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
+    if ((rc = start_build(ctx))) return rc;
     HIPCHK(hipMemsetAsync(d_gC, 0, ctx->nnz * sizeof(double), ctx->stream));
     if (d_gB) HIPCHK(hipMemsetAsync(d_gB, 0, ctx->nnzB * sizeof(double), ctx->stream));
     BuildArgs a = base_args(ctx);
@@ -1799,27 +1876,18 @@ extern "C" int mspai_backward(mspai_ctx* ctx, const mspai_opts* opts, const doub
     a.gC = d_gC;
     a.gB = d_gB;
     a.cap = cap;
-    HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
     int first = -1;
     if (opts->binning) {
         if ((rc = run_static(ctx, a, wide, G, gwaves, 2, opts->precision == 1, n, cap, (double)ctx->nnzM / n, &first))) return rc;
     } else {
-        if ((rc = run_chain(ctx, a, wide, wide, G, gwaves, false, 2, n))) return rc;
+        if ((rc = run_chain(ctx, a, wide, wide, G, gwaves, false, 2, n, cap))) return rc;
     }
-    HIPCHK(hipEventRecord(ctx->ev[2], ctx->stream));
-    HIPCHK(hipEventRecord(ctx->ev[3], ctx->stream));
+    hipLaunchKernelGGL(stamp_kernel, dim3(1), dim3(1), 0, ctx->stream, ctx->d_ts + kStampSolved);
     if ((rc = fetch_counters(ctx))) return rc;
     HIPCHK(hipStreamSynchronize(ctx->stream));
     if (stats) {
         std::memset(stats, 0, sizeof(*stats));
-        float t_all = 0, t_solve = 0;
-        HIPCHK(hipEventElapsedTime(&t_all, ctx->ev[0], ctx->ev[3]));
-        float t_first = 0;
-        HIPCHK(hipEventElapsedTime(&t_first, ctx->ev[4], ctx->ev[5]));
-        stats->first_bin_ms = t_first;
-        HIPCHK(hipEventElapsedTime(&t_solve, ctx->ev[1], ctx->ev[2]));
-        stats->build_ms = t_all;
-        stats->solve_ms = t_solve;
+        build_times(ctx, stats);
         stats->nnz = ctx->nnz;
         stats->ncols = n;
         if (first >= 0) ctx->h_counter[first] = ctx->h_counter[16 + first] = n;  // not through a queue
@@ -1914,9 +1982,7 @@ extern "C" int mspai_launch_stats(mspai_ctx* ctx, int max, int* nlaunch, mspai_l
         mspai_launch_stat& o = out[k];
         std::memset(&o, 0, sizeof o);
         std::snprintf(o.name, sizeof o.name, "%s", ctx->lname[k]);
-        float ms = 0;
-        HIPCHK(hipEventElapsedTime(&ms, ctx->lev[2 * k], ctx->lev[2 * k + 1]));
-        o.ms = ms;
+        o.ms = launch_ms(ctx, k);
         const double* t = tot.data() + (size_t)k * kLaunchStat;
         for (int q = 0; q < kNumWork; ++q) o.work[q] = t[q];
         o.columns = t[kNumWork];

@@ -102,9 +102,8 @@ struct BuildArgs {
     int maxnew, ns, use_mean;
     int cap;                // capacity of one output column
     int direct;             // static build: column k's outputs at p_ptr[k] (M has the start pattern) instead of k*cap
-    const int* queue;       // columns to build in this launch
-    int nqueue;
-    int* counter;           // persistent work-queue head
+    int nqueue;             // columns 0..nqueue of a launch without a queue
+    unsigned long long* stamp;  // start time of this launch
     int* overflow;          // columns that did not fit this launch's layout
     int* n_overflow;        // their count
     int* fallback;          // mixed path: columns to rebuild in FP64

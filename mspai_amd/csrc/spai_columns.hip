@@ -2583,7 +2583,7 @@ __device__ __forceinline__ void save_column_state(const BuildArgs& a, const Wave
 
 template <int G, bool kMixed, int NMAX, bool kTies, bool kTail = false>
 __device__ __forceinline__ int solve_column(const BuildArgs& a, const ScratchLayout& L, const WaveScratch& s,
-                                            int col)
+                                            int col, bool fresh)
 {
     /* NMAX 20 or 24 in a 64-lane bin: the row-group register QR with eight
      * rows per lane (|I| <= 128, FP64 builds) */
@@ -2594,7 +2594,7 @@ __device__ __forceinline__ int solve_column(const BuildArgs& a, const ScratchLay
     int st = 0, step0 = -1, n;
     int near[3] = {0, 0, 0};  // near-margin decisions (counters builds, FP64)
     const size_t o = output_slot(a, col);
-    const int mark = a.nsolve[col];
+    const int mark = fresh ? 0 : a.nsolve[col];  // fresh: not routed, no launch has seen the column
     const int* jsrc;
     if (mark < 0) {
         /* resume the state an earlier launch of this precision left at the
@@ -2768,7 +2768,8 @@ __global__ __launch_bounds__(64, kWaves > 0 ? kWaves
      * budget spills of them would otherwise be stored by every wave.  The
      * length does not change during the launch (waves append to other
      * queues only). */
-    const int nq = *nqueue;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *a.stamp = wall_clock64();
+    const int nq = queue ? *nqueue : a.nqueue;
     if (nq <= 0) return;
     constexpr int NG = kWave / G;
     const int g = Group<G>::index();
@@ -2823,9 +2824,9 @@ __global__ __launch_bounds__(64, kWaves > 0 ? kWaves
             int col = -1;
             int outcome = kDone;
             if (q < nq) {
-                col = queue[q];
+                col = queue ? queue[q] : (int)q;
                 if (kMode < 2)
-                    outcome = solve_column<G, kMode == 1, NMAX, !kLds, kWaves == 1>(a, L, s, col);
+                    outcome = solve_column<G, kMode == 1, NMAX, !kLds, kWaves == 1>(a, L, s, col, !queue);
                 else if (kMode == 2)
                     outcome = backward_column<G, !kLds>(a, L, s, col);
                 else
@@ -2884,6 +2885,7 @@ __global__ __launch_bounds__(kClassifyBlock) void classify_kernel(BuildArgs a, i
                                                        int* counts, int* gqueue, int* gcount, int n, int* done,
                                                        int* routed)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *a.stamp = wall_clock64();
     int col = blockIdx.x * blockDim.x + threadIdx.x;
     int bin = nbins;  // generic
     if (col < n) {

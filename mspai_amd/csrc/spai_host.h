@@ -15,7 +15,8 @@ namespace mspai {
  * that do not fit go to a.overflow.  mode 0: FP64 build; 1: FP32 QR + FP64
  * refinement, columns whose selection margins are too small go to
  * a.fallback; 2/3: the adjoint in FP64 / mixed; 4: FP64 build with the
- * dense QR update (-qr 2). */
+ * dense QR update (-qr 2).  Without a queue (nullptr): columns
+ * 0..a.nqueue, none seen by an earlier launch of the build. */
 void launch_binned(const BuildArgs& a, const ScratchLayout& L, int group, int mode, const int* queue,
                    const int* nqueue, int* head, int nwaves, hipStream_t stream, int wcap = 0);
 
@@ -46,14 +47,14 @@ void launch_fp64_generic(const BuildArgs& a, const ScratchLayout& L, int mode, c
 constexpr int kStaticKinds = 3;
 constexpr int kStaticJ[kStaticKinds] = {7, 15, 31};
 constexpr int kStaticI[kStaticKinds] = {32, 64, 64};
-void launch_static_columns(int kind, const BuildArgs& a, bool back, bool refine, const int* queue, const int* nqueue, int nall,
-                           int num_cu, hipStream_t stream);
-/* colptr, rowind and *count (entries) of an M that has the start pattern. */
+void launch_static_columns(int kind, const BuildArgs& a, bool back, bool refine, const int* queue, const int* nqueue,
+                           int nall, int num_cu, hipStream_t stream);
+/* colptr, rowind and *count (entries) of an M that has the start pattern;
+ * *stamp: the time this kernel starts. */
 void launch_copy_pattern(int ncols, int nnz, const int* p_ptr, const int* p_ind, int* colptr, int* rowind,
-                         int* count, hipStream_t stream);
+                         int* count, unsigned long long* stamp, hipStream_t stream);
 
 /* Sparse products (apply.hip). */
-void launch_fill_int(int* p, long long count, int value, hipStream_t stream);
 /* col_of[e] = column of CSC entry e, order[e] = e. */
 void launch_csr_entry_cols(const int* colptr, int ncols, int* col_of, int* order, hipStream_t stream);
 /* rowptr[0..nrows] from the row indices of the entries sorted by row. */

@@ -636,6 +636,7 @@ __global__ __launch_bounds__(64, kWaves) void static_column_kernel(BuildArgs a, 
     using W = StaticLds<CG, S, KR>;
     constexpr int NG = kWave / W::G;
     __shared__ W work[NG];
+    if (blockIdx.x == 0 && threadIdx.x == 0) *a.stamp = wall_clock64();
     const int nq = queue ? *nqueue : nall;
     const int g = (int)threadIdx.x / W::G;
     /* workgroups go round-robin to the 8 XCDs: XCD x takes the x-th
@@ -655,8 +656,9 @@ __global__ __launch_bounds__(64, kWaves) void static_column_kernel(BuildArgs a, 
 /* M of a static build has the start pattern: its column pointers, indices
  * and number of entries. */
 __global__ __launch_bounds__(256) void copy_pattern_kernel(int ncols, int nnz, const int* p_ptr, const int* p_ind,
-                                                          int* colptr, int* rowind, int* count)
+                                                          int* colptr, int* rowind, int* count, unsigned long long* stamp)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *stamp = wall_clock64();
     const int stride = (int)(gridDim.x * blockDim.x);
     const int t0 = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     for (int t = t0; t <= ncols; t += stride) colptr[t] = p_ptr[t];
@@ -665,8 +667,8 @@ __global__ __launch_bounds__(256) void copy_pattern_kernel(int ncols, int nnz, c
 }
 
 template <int CG, int S, int KR, int kWaves>
-void launch_kind(const BuildArgs& a, bool back, bool refine, const int* queue, const int* nqueue, int nall, int num_cu,
-                 hipStream_t stream)
+void launch_kind(const BuildArgs& a, bool back, bool refine, const int* queue, const int* nqueue, int nall,
+                 int num_cu, hipStream_t stream)
 {
     constexpr int NG = kWave / (4 * CG);
     const long long all = ((long long)nall + NG - 1) / NG;
@@ -683,8 +685,8 @@ void launch_kind(const BuildArgs& a, bool back, bool refine, const int* queue, c
 
 }  // namespace
 
-void launch_static_columns(int kind, const BuildArgs& a, bool back, bool refine, const int* queue, const int* nqueue, int nall,
-                           int num_cu, hipStream_t stream)
+void launch_static_columns(int kind, const BuildArgs& a, bool back, bool refine, const int* queue, const int* nqueue,
+                           int nall, int num_cu, hipStream_t stream)
 {
     switch (kind) {
     case 0: launch_kind<2, 4, 8, 3>(a, back, refine, queue, nqueue, nall, num_cu, stream); break;
@@ -694,12 +696,12 @@ void launch_static_columns(int kind, const BuildArgs& a, bool back, bool refine,
 }
 
 void launch_copy_pattern(int ncols, int nnz, const int* p_ptr, const int* p_ind, int* colptr, int* rowind,
-                         int* count, hipStream_t stream)
+                         int* count, unsigned long long* stamp, hipStream_t stream)
 {
     const long long t = std::max<long long>(nnz, ncols + 1);
     const unsigned grid = (unsigned)std::min<long long>((t + 255) / 256, 4096);
     hipLaunchKernelGGL(copy_pattern_kernel, dim3(grid), dim3(256), 0, stream, ncols, nnz, p_ptr, p_ind, colptr,
-                       rowind, count);
+                       rowind, count, stamp);
 }
 
 }  // namespace mspai
