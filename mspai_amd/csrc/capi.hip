@@ -1030,69 +1030,69 @@ static const BinTable kTables[] = {
     {"g32-g64-g64/occ8", 3, {{32, 16, 32, 128, 256, 8}, {64, 32, 64, 256, 512, 0}, {64, 40, 128, 512, 1024, 0}}},
     {"g16-g64/occ10", 2, {{16, 8, 16, 64, 128, 10}, {64, 40, 128, 512, 1024, 0}}},
     /* long candidate lists: a last bin of |I| <= 384 and raw lists to 8192
-     * (about 117 KB of LDS per wave at |J| <= 33, one wave per CU) keeps the
-     * widest columns of the random band out of the HBM working set */
+     * (a workgroup of eight waves per column, one per CU) keeps the widest
+     * columns of the random band out of the HBM working set */
     {"g16-g64-g64-g64x384", 4,
      {{16, 8, 16, 64, 128, 0}, {64, 32, 64, 512, 1024, 0}, {64, 40, 128, 1024, 2048, 0},
-      {64, 40, 384, 4096, 8192, 0}}},
+      {512, 40, 384, 4096, 8192, 0}}},
     {"g16-g64-g64x192-g64x384", 4,
      {{16, 8, 16, 64, 128, 0}, {64, 32, 64, 512, 1024, 0}, {64, 40, 192, 2048, 4096, 0},
-      {64, 40, 384, 4096, 8192, 0}}},
+      {512, 40, 384, 4096, 8192, 0}}},
     {"g32-g64-g64-g64x384", 4,
      {{32, 16, 32, 256, 512, 0}, {64, 32, 64, 512, 1024, 0}, {64, 40, 128, 1024, 2048, 0},
-      {64, 40, 384, 4096, 8192, 0}}},
+      {512, 40, 384, 4096, 8192, 0}}},
     {"g64-g64-g64x384", 3,
-     {{64, 32, 64, 512, 1024, 0}, {64, 40, 128, 1024, 2048, 0}, {64, 40, 384, 4096, 8192, 0}}},
+     {{64, 32, 64, 512, 1024, 0}, {64, 40, 128, 1024, 2048, 0}, {512, 40, 384, 4096, 8192, 0}}},
     /* no size bins: every column in the generic kernel */
     {"generic", 0, {}},
     /* |J| <= 16 in the bulk bin: half the A(I,J) region, about 14 KB of LDS
      * per wave, 11 resident waves per CU instead of 7 */
     {"g64x16-g64-g64x384", 3,
-     {{64, 16, 64, 512, 1024, 0}, {64, 40, 128, 1024, 2048, 0}, {64, 40, 384, 4096, 8192, 0}}},
+     {{64, 16, 64, 512, 1024, 0}, {64, 40, 128, 1024, 2048, 0}, {512, 40, 384, 4096, 8192, 0}}},
     {"g16-g64x16-g64-g64x384", 4,
      {{16, 8, 16, 64, 128, 0}, {64, 16, 64, 512, 1024, 0}, {64, 40, 128, 1024, 2048, 0},
-      {64, 40, 384, 4096, 8192, 0}}},
+      {512, 40, 384, 4096, 8192, 0}}},
     /* the same with the bulk bin at 8 resident waves per CU: its FP64
      * kernel then keeps every register (no spills to scratch) */
     {"g64x16/occ8-g64-g64x384", 3,
-     {{64, 16, 64, 512, 1024, 8}, {64, 40, 128, 1024, 2048, 0}, {64, 40, 384, 4096, 8192, 0}}},
+     {{64, 16, 64, 512, 1024, 8}, {64, 40, 128, 1024, 2048, 0}, {512, 40, 384, 4096, 8192, 0}}},
     {"g16-g64x16/occ8-g64-g64x384", 4,
      {{16, 8, 16, 64, 128, 0}, {64, 16, 64, 512, 1024, 8}, {64, 40, 128, 1024, 2048, 0},
-      {64, 40, 384, 4096, 8192, 0}}},
+      {512, 40, 384, 4096, 8192, 0}}},
     /* a narrower second bin (|J| <= 24 or 20, |I| <= 96 or 112: about 26 KB,
      * 6 resident waves per CU instead of 3) ahead of the wide ones */
     {"g64x16-g64x24i96-g64i160-g64x384", 4,
      {{64, 16, 64, 512, 1024, 0}, {64, 24, 96, 1024, 2048, 0}, {64, 40, 160, 2048, 4096, 0},
-      {64, 40, 384, 4096, 8192, 0}}},
+      {512, 40, 384, 4096, 8192, 0}}},
     {"g64x16-g64x24i96-g64x384", 3,
-     {{64, 16, 64, 512, 1024, 0}, {64, 24, 96, 1024, 2048, 0}, {64, 40, 384, 4096, 8192, 0}}},
+     {{64, 16, 64, 512, 1024, 0}, {64, 24, 96, 1024, 2048, 0}, {512, 40, 384, 4096, 8192, 0}}},
     {"g64x16-g64x20i112-g64x384", 3,
-     {{64, 16, 64, 512, 1024, 0}, {64, 20, 112, 1024, 2048, 0}, {64, 40, 384, 4096, 8192, 0}}},
+     {{64, 16, 64, 512, 1024, 0}, {64, 20, 112, 1024, 2048, 0}, {512, 40, 384, 4096, 8192, 0}}},
     /* the same two with the FP32 QR in the bulk bin only: the wider bins'
      * FP64 kernels run faster than their mixed ones (identical tables in
      * FP64 builds, which the autotuner skips) */
     {"g64x16-g64x24i96-g64x384/m1", 3,
-     {{64, 16, 64, 512, 1024, 0}, {64, 24, 96, 1024, 2048, 0}, {64, 40, 384, 4096, 8192, 0}}, 1},
+     {{64, 16, 64, 512, 1024, 0}, {64, 24, 96, 1024, 2048, 0}, {512, 40, 384, 4096, 8192, 0}}, 1},
     {"g64x16-g64x20i112-g64x384/m1", 3,
-     {{64, 16, 64, 512, 1024, 0}, {64, 20, 112, 1024, 2048, 0}, {64, 40, 384, 4096, 8192, 0}}, 1},
+     {{64, 16, 64, 512, 1024, 0}, {64, 20, 112, 1024, 2048, 0}, {512, 40, 384, 4096, 8192, 0}}, 1},
     /* (u) the bulk bin with room for 384 candidates instead of 512: about
      * 1.5 KB less LDS per wave, one more resident wave per CU */
     {"g64x16u-g64x20i112-g64x384", 3,
-     {{64, 16, 64, 384, 1024, 0}, {64, 20, 112, 1024, 2048, 0}, {64, 40, 384, 4096, 8192, 0}}},
+     {{64, 16, 64, 384, 1024, 0}, {64, 20, 112, 1024, 2048, 0}, {512, 40, 384, 4096, 8192, 0}}},
     {"g64x16u-g64x20i112-g64x384/m1", 3,
-     {{64, 16, 64, 384, 1024, 0}, {64, 20, 112, 1024, 2048, 0}, {64, 40, 384, 4096, 8192, 0}}, 1},
+     {{64, 16, 64, 384, 1024, 0}, {64, 20, 112, 1024, 2048, 0}, {512, 40, 384, 4096, 8192, 0}}, 1},
     /* a second bin of |J| <= 24, |I| <= 128 (the eight-row register QR),
      * alone or after the |J| <= 20, |I| <= 112 one */
     {"g64x16u-g64x24i128-g64x384", 3,
-     {{64, 16, 64, 384, 1024, 0}, {64, 24, 128, 1024, 2048, 0}, {64, 40, 384, 4096, 8192, 0}}},
+     {{64, 16, 64, 384, 1024, 0}, {64, 24, 128, 1024, 2048, 0}, {512, 40, 384, 4096, 8192, 0}}},
     {"g64x16u-g64x24i128-g64x384/m1", 3,
-     {{64, 16, 64, 384, 1024, 0}, {64, 24, 128, 1024, 2048, 0}, {64, 40, 384, 4096, 8192, 0}}, 1},
+     {{64, 16, 64, 384, 1024, 0}, {64, 24, 128, 1024, 2048, 0}, {512, 40, 384, 4096, 8192, 0}}, 1},
     {"g64x16u-x20i112-x24i128-x384", 4,
      {{64, 16, 64, 384, 1024, 0}, {64, 20, 112, 1024, 2048, 0}, {64, 24, 128, 1024, 2048, 0},
-      {64, 40, 384, 4096, 8192, 0}}},
+      {512, 40, 384, 4096, 8192, 0}}},
     {"g64x16u-x20i112-x24i128-x384/m1", 4,
      {{64, 16, 64, 384, 1024, 0}, {64, 20, 112, 1024, 2048, 0}, {64, 24, 128, 1024, 2048, 0},
-      {64, 40, 384, 4096, 8192, 0}}, 1},
+      {512, 40, 384, 4096, 8192, 0}}, 1},
     /* mixed builds: FP32 in the bulk bin and (the Gram matrix on the matrix
      * cores) in the widest one, the second bin in FP64 on its eight-row
      * register QR (f) */
@@ -1113,7 +1113,22 @@ static std::vector<Bin> bin_layouts(const mspai_ctx* ctx, int cap, int maxnew, b
     std::vector<Bin> out;
     for (int t = 0; t < table.count; ++t) {
         if ((needs & kNeedMixed) && table.mixed > 0 && (int)out.size() >= table.mixed) break;
-        const BinEdge& e = table.e[t];
+        BinEdge e = table.e[t];
+        if (e.group == kWideGroup) {
+            /* one column per workgroup in FP64 (also in a mixed build's
+             * chain); the QR update has one-wave kernels only */
+            if (needs & kNeedQrUpdate) {
+                e.group = kWave;
+            } else {
+                if (wide_lds_bytes() > ctx->lds_block) continue;
+                ScratchLayout L = make_layout(std::min(cap, kWideJ), std::min<size_t>(G.capI, kWideI), kWideU, kWideRaw,
+                                              maxnew, 1, needs & ~kNeedMixed, false, kWave);
+                L.per_wave = wide_lds_bytes();
+                L.tie_per_group = 0;
+                out.push_back({kWideGroup, e.wcap, L, (needs & kNeedMixed) != 0});
+                continue;
+            }
+        }
         int capJ = std::min(cap, e.J);
         size_t capI = std::min<size_t>(G.capI, e.I);
         size_t capU = adaptive ? std::min<size_t>(G.capU, e.U) : 1;
@@ -1155,6 +1170,7 @@ static int ensure_scratch(mspai_ctx* ctx, size_t need)
  * waves that find the queue drained. */
 static int waves_per_cu(const Bin& b, int mode)
 {
+    if (b.group == kWideGroup) return 1;  // workgroups: LDS holds one
     size_t lds = b.L.per_wave * (64 / b.group);
     int w = (int)std::min<size_t>(32, std::max<size_t>(1, (160 * 1024) / lds));
     const int occ = binned_blocks_per_cu(b.L, b.group, mode, b.wcap);

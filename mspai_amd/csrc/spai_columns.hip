@@ -3027,6 +3027,10 @@ int binned_blocks_per_cu(const ScratchLayout& L, int group, int mode, int wcap)
 void launch_binned(const BuildArgs& a, const ScratchLayout& L, int group, int mode, const int* queue,
                    const int* nqueue, int* head, int nwaves, hipStream_t stream, int wcap)
 {
+    if (group == kWideGroup) {
+        launch_wide(a, queue, nqueue, head, nwaves, stream);
+        return;
+    }
     const size_t lds = L.per_wave * (kWave / group);
     hipLaunchKernelGGL(binned_kernel(L, group, mode, wcap), dim3(nwaves), dim3(kWave), lds, stream, a, L, queue, nqueue,
                        head);

@@ -39,6 +39,15 @@ void launch_copy_ints(const int* src, int* dst, int count, hipStream_t stream);
 void launch_fp64_generic(const BuildArgs& a, const ScratchLayout& L, int mode, const int* queue,
                          const int* nqueue, int* head, int nwaves, hipStream_t stream);
 
+/* FP64 adaptive kernel with one column per workgroup of eight waves
+ * (spai_wide.hip): |J| <= kWideJ, |I| <= kWideI, kWideU candidates out of raw
+ * lists of kWideRaw; other columns go to a.overflow.  kWideGroup is its lane
+ * count, the group width of its size bin. */
+constexpr int kWideGroup = 512;
+constexpr int kWideJ = 40, kWideI = 384, kWideU = 4096, kWideRaw = 8192;
+size_t wide_lds_bytes();
+void launch_wide(const BuildArgs& a, const int* queue, const int* nqueue, int* head, int blocks, hipStream_t stream);
+
 /* Column kernels for a given pattern (spai_static.hip): static FP64 build, or
  * with `back` the adjoint.  Kind k takes columns of |J| <= kStaticJ[k] and
  * |I| <= kStaticI[k]: those of queue (length *nqueue), or without a queue all
