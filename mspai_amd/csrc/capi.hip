@@ -25,7 +25,7 @@
 
 using namespace mspai;
 
-constexpr int kMaxBins = 4;
+constexpr int kMaxBins = 5;
 constexpr int kMaxLaunch = 2 * kMaxBins + 2;  // column-kernel launches of one build: mixed bins, FP64 bins, generic
 /* Time stamps of a build, written by the kernels themselves as they start (an
  * event between two launches holds the stream for several microseconds): one
@@ -297,6 +297,7 @@ struct mspai_ctx {
     int tuned_table[2] = {-1, -1};  // autotuner's choice for this matrix (binning == 2), FP64 and mixed
     int last_table = 0;
     int last_nbins = 0;
+    unsigned long long first_end = 0;  // end of the first launch when the host looked at its counters (else 0)
     bool last_mixed = false;
     int last_binning = 1;
     bool last_counters = false;  // the last build stored per-column work counters
@@ -1007,16 +1008,17 @@ struct BinEdge {
 struct BinTable {
     const char* name;
     int count;
-    BinEdge e[4];
+    BinEdge e[kMaxBins];
     int mixed;
     int fp64mask;  // bins (bit t for entry t) that a mixed build runs in FP64 inside its chain
 };
 
-/* Candidate tables of the autotuner; table 0 is the default. */
+/* Candidate tables of the autotuner; default_table says which one an untuned
+ * build takes. */
 static const BinTable kTables[] = {
-    {"g16-g32-g64-g64", 4,
+    {"g16-g32-g64-g64-g64x384", 5,
      {{16, 8, 16, 64, 128, 0}, {32, 16, 32, 128, 256, 0}, {64, 32, 64, 256, 512, 0},
-      {64, 40, 128, 512, 1024, 0}}},
+      {64, 40, 128, 512, 1024, 0}, {512, 40, 384, 4096, 8192, 0}}},
     {"g32-g64-g64", 3,
      {{32, 16, 32, 128, 256, 0}, {64, 32, 64, 256, 512, 0}, {64, 40, 128, 512, 1024, 0}}},
     {"g16wide-g64-g64", 3,
@@ -1146,12 +1148,37 @@ static std::vector<Bin> bin_layouts(const mspai_ctx* ctx, int cap, int maxnew, b
     return out;
 }
 
+/* Entries of the row patterns that a column's first candidate list gathers,
+ * on average: |J0| columns of A, a row of A for each of their entries. */
+static double mean_first_list(const mspai_ctx* ctx)
+{
+    const double col = (double)ctx->nnz / ctx->ncols, row = (double)ctx->nnz / ctx->nrows;
+    return (double)ctx->p_nnz / ctx->ncols * col * row;
+}
+
+/* The table of an untuned build.  Where the average column's first candidate
+ * list already outgrows the 16- and 32-lane bins of table 0 (128 candidates in
+ * the wider one), those bins would build every column's first step and pass
+ * it on, and most columns would pass the narrow 64-lane bins as well: the
+ * chain then begins with the 64-lane bulk bin.  The random band (12 entries
+ * a row, lists of 144, n = 262,144, FP64): 5.3 ms instead of 12.6 ms.  The 2D
+ * grid operators (5 entries, lists of 25) stay in the 16-lane bin: 0.24 ms on
+ * the 256^2 grid in FP64 and 0.50 ms on the 371^2 one mixed, against 0.79 and
+ * 1.94 ms with the chain that begins wide. (The QR
+ * update's bins do not hold the wide chain's sizes.) */
+constexpr int kWideFp64 = 25, kWideMixed = 26;  // g64x16u-g64x24i128-g64x384 and its /m1
+static int default_table(const mspai_ctx* ctx, const mspai_opts* o)
+{
+    const bool wide = o->max_impr_steps > 0 && o->qr != 2 && mean_first_list(ctx) > 128.0;
+    return !wide ? 0 : o->precision == 1 ? kWideMixed : kWideFp64;
+}
+
 /* The bin table of a build: the autotuner's choice for the build's precision
- * (binning == 2), else table 0. */
+ * (binning == 2), else the default. */
 static int table_for(const mspai_ctx* ctx, const mspai_opts* o)
 {
     const int t = ctx->tuned_table[o->precision == 1 ? 1 : 0];
-    return o->binning == 2 && t >= 0 ? t : 0;
+    return o->binning == 2 && t >= 0 ? t : default_table(ctx, o);
 }
 
 static int ensure_scratch(mspai_ctx* ctx, size_t need)
@@ -1204,6 +1231,7 @@ static int start_build(mspai_ctx* ctx)
     HIPCHK(hipGetLastError());
     ctx->nlaunch = 0;
     ctx->was_routed = false;
+    ctx->first_end = 0;
     return MSPAI_OK;
 }
 
@@ -1215,6 +1243,7 @@ static double stamp_ms(const mspai_ctx* ctx, int from, int to)
 /* Duration of column-kernel launch k of the last build. */
 static double launch_ms(const mspai_ctx* ctx, int k)
 {
+    if (k == 0 && ctx->first_end) return (double)(ctx->first_end - ctx->h_ts[0]) / ctx->ticks_per_ms;
     return stamp_ms(ctx, k, k + 1 < ctx->nlaunch ? k + 1 : kStampSolved);
 }
 
@@ -1244,6 +1273,21 @@ static size_t tie_bytes_needed(const mspai_ctx* ctx, const std::vector<Bin>& bin
 /* Most FP64 columns of a mixed build that the generic kernel takes alone. */
 constexpr int kDirectFp64 = 4096;
 
+/* No start pattern (at most `longest` indices) can outgrow the first bin of
+ * the chain, |J0| and rows being at most their entries: the bin takes all
+ * columns by index and the routing kernel is not run (70 us of 0.26 million
+ * columns, 22 us of 65 thousand). */
+static bool straight_chain(const mspai_ctx* ctx, const std::vector<Bin>& routed, int fp64_mode, int longest)
+{
+    const size_t raw = (size_t)longest * ctx->maxcolnnz;
+    return fp64_mode == 0 && !routed.empty() && longest <= routed[0].L.capJ &&
+           raw <= (size_t)std::min(routed[0].L.capI, routed[0].L.capSid);
+}
+
+/* What run_chain launches: the whole chain, its first bin (of a straight
+ * chain), or what follows that. */
+enum ChainPart { kWholeChain, kFirstBin, kRestOfChain };
+
 /* Launch routing and the bin chain over the columns whose patterns are in
  * a.p_ptr/p_ind.  `bins` are the mixed chain's bins in a mixed build (else
  * the FP64 chain's), `fbins` the FP64 chain's.  Queues: FP64 queue b at
@@ -1256,7 +1300,8 @@ constexpr int kDirectFp64 = 4096;
  * [8..16) heads, [16..24) routed lengths, mixed [24..32) lengths, [32..40)
  * heads, [40] blocks of the routing kernel done. */
 static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins, const std::vector<Bin>& fbins,
-                     const ScratchLayout& G, int gwaves, bool mixed, int fp64_mode, int n, int longest)
+                     const ScratchLayout& G, int gwaves, bool mixed, int fp64_mode, int n, int longest,
+                     ChainPart part = kWholeChain)
 {
     const int nb = (int)bins.size();
     const int nf = (int)fbins.size();
@@ -1267,13 +1312,7 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
         edges.capSort[b] = routed[b].L.capSid;  // the I-set raw list of the start pattern
         edges.capI[b] = routed[b].L.capI;
     }
-    /* when no start pattern can outgrow the first bin (|J0| at most `longest`,
-     * rows at most their entries), the bin takes all columns by index and the
-     * routing kernel is not run (70 us of 0.26 million columns, 22 us of 65
-     * thousand) */
-    const size_t raw = (size_t)longest * ctx->maxcolnnz;
-    const bool straight = fp64_mode == 0 && !routed.empty() && longest <= routed[0].L.capJ &&
-                          raw <= (size_t)std::min(routed[0].L.capI, routed[0].L.capSid);
+    const bool straight = straight_chain(ctx, routed, fp64_mode, longest);
     ctx->was_routed = !straight;
     a.nqueue = n;
     int* counts = ctx->d_counter;
@@ -1318,7 +1357,7 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
         HIPCHK(hipGetLastError());
         a.fallback = fq;
         a.n_fallback = counts;
-        for (int b = 0; b < nb; ++b) {
+        for (int b = part == kRestOfChain ? 1 : 0; b < nb; ++b) {
             const int grp = bins[b].group;
             a.overflow = b + 1 < nb ? mq + (size_t)(b + 1) * n : fq + (size_t)to * n;
             /* overflow and declined steps go on from the step they reached,
@@ -1334,6 +1373,7 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
             launch_binned(a, L, grp, mode, straight && b == 0 ? nullptr : mq + (size_t)b * n, mcounts + b, mheads + b, ctx->num_cu * per_cu,
                           ctx->stream, bins[b].wcap);
             HIPCHK(hipGetLastError());
+            if (part == kFirstBin) return MSPAI_OK;
         }
         a.status_or = COL_FALLBACK;
         a.save_state = 0;
@@ -1356,7 +1396,7 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
     }
     a.fallback = nullptr;
     a.n_fallback = nullptr;
-    for (int b = 0; b < nf; ++b) {
+    for (int b = part == kRestOfChain && !mixed ? 1 : 0; b < nf; ++b) {
         const int grp = fbins[b].group;
         a.overflow = fq + (size_t)(b + 1) * n;
         a.n_overflow = counts + b + 1;
@@ -1368,6 +1408,7 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
                       heads + b,
                       ctx->num_cu * per_cu, ctx->stream, fbins[b].wcap);
         HIPCHK(hipGetLastError());
+        if (part == kFirstBin) return MSPAI_OK;
     }
     a.overflow = fq;  // never written: the generic layout holds every column
     a.n_overflow = counts + 7;
@@ -1664,29 +1705,57 @@ extern "C" int mspai_build(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* 
         a.cache_hits = ctx->d_counter + 48;
     }
     int first = -1;
-    if (given) {
-        if ((rc = run_static(ctx, a, bins, G, gwaves, 0, opts->precision == 1, n, ctx->plen_max, (double)ctx->p_nnz / n, &first))) return rc;
-    } else {
-        if ((rc = run_chain(ctx, a, bins, fbins, G, gwaves, mixed, qrup ? 4 : 0, n,
-                            ctx->plen_max)))
-            return rc;
-    }
     unsigned long long* const solved = ctx->d_ts + kStampSolved;
     if (given) {
+        if ((rc = run_static(ctx, a, bins, G, gwaves, 0, opts->precision == 1, n, ctx->plen_max, (double)ctx->p_nnz / n, &first))) return rc;
         launch_copy_pattern(n, ctx->p_nnz, ctx->d_p_ptr, ctx->d_p_ind, ctx->d_Mptr, ctx->d_Mind,
                             ctx->d_counter + 63, solved, ctx->stream);
+        HIPCHK(hipGetLastError());
+        if ((rc = fetch_counters(ctx))) return rc;
+        HIPCHK(hipStreamSynchronize(ctx->stream));
     } else {
-        /* the queues are empty now: the tiles' sums go there */
-        const int tiles = (n + kTileCols - 1) / kTileCols;
-        hipLaunchKernelGGL(tile_sums_kernel, dim3(tiles), dim3(kTileCols), 0, ctx->stream, n, ctx->d_m_len,
-                           mixed ? ctx->d_status : nullptr, COL_FALLBACK, ctx->d_queues, ctx->d_counter + 62, solved);
-        hipLaunchKernelGGL(compact_columns_kernel, dim3(tiles), dim3(kTileCols), 0, ctx->stream, n, cap,
-                           ctx->d_m_len, ctx->d_m_idx, ctx->d_m_val, ctx->d_queues, ctx->d_Mptr, ctx->d_Mind,
-                           ctx->d_Mval, ctx->d_counter + 63);
+        const std::vector<Bin>& routed = mixed ? bins : fbins;
+        const int fp64_mode = qrup ? 4 : 0;
+        /* M's columns from the slots, counters to the host */
+        auto finish = [&](int* tile_sum) -> int {
+            const int tiles = (n + kTileCols - 1) / kTileCols;
+            hipLaunchKernelGGL(tile_sums_kernel, dim3(tiles), dim3(kTileCols), 0, ctx->stream, n, ctx->d_m_len,
+                               mixed ? ctx->d_status : nullptr, COL_FALLBACK, tile_sum, ctx->d_counter + 62, solved);
+            hipLaunchKernelGGL(compact_columns_kernel, dim3(tiles), dim3(kTileCols), 0, ctx->stream, n, cap,
+                               ctx->d_m_len, ctx->d_m_idx, ctx->d_m_val, tile_sum, ctx->d_Mptr, ctx->d_Mind,
+                               ctx->d_Mval, ctx->d_counter + 63);
+            HIPCHK(hipGetLastError());
+            if (const int e = fetch_counters(ctx)) return e;
+            HIPCHK(hipStreamSynchronize(ctx->stream));
+            return MSPAI_OK;
+        };
+        /* where the first candidate lists fill a quarter of the first bin on
+         * average, it most likely holds every column to its end: M is
+         * assembled right after it, and only if the counters then show a
+         * column that moved on do the other launches of the chain (5 on empty
+         * queues in FP64, 10 mixed: 21 and 33 us on the 256^2 and 371^2 grids)
+         * and a second assembly follow (about 40 us).  Not with counters, whose launches are all listed. */
+        const bool alone = !a.work && straight_chain(ctx, routed, fp64_mode, ctx->plen_max) &&
+                           4.0 * mean_first_list(ctx) <= routed[0].L.capSort;
+        if ((rc = run_chain(ctx, a, bins, fbins, G, gwaves, mixed, fp64_mode, n, ctx->plen_max,
+                            alone ? kFirstBin : kWholeChain)))
+            return rc;
+        /* the tiles' sums go to a queue that is empty: the first one, or with
+         * the chain not ended the mixed one that the straight chain leaves */
+        int* const sums = ctx->d_queues + (alone && mixed ? (size_t)(kMaxBins + 1) * n : 0);
+        if ((rc = finish(sums))) return rc;
+        const int* hc = ctx->h_counter;
+        int moved = 0;
+        for (int b = 0; alone && b < 8; ++b) moved += hc[b] + hc[24 + b];
+        if (moved) {
+            ctx->first_end = ctx->h_ts[kStampSolved];
+            /* the column count of the first assembly is taken back */
+            hipLaunchKernelGGL(start_kernel, dim3(1), dim3(1), 0, ctx->stream, ctx->d_counter + 62, solved);
+            if ((rc = run_chain(ctx, a, bins, fbins, G, gwaves, mixed, fp64_mode, n, ctx->plen_max, kRestOfChain)))
+                return rc;
+            if ((rc = finish(ctx->d_queues))) return rc;
+        }
     }
-    HIPCHK(hipGetLastError());
-    if ((rc = fetch_counters(ctx))) return rc;
-    HIPCHK(hipStreamSynchronize(ctx->stream));
 
     const int last = ctx->h_counter[63];
     ctx->nnzM = last;
