@@ -1729,13 +1729,13 @@ extern "C" int mspai_build(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* 
             HIPCHK(hipStreamSynchronize(ctx->stream));
             return MSPAI_OK;
         };
-        /* where the first candidate lists fill a quarter of the first bin on
-         * average, it most likely holds every column to its end: M is
+        /* where the first candidate lists fill a quarter of a 16- or 32-lane
+         * first bin on average, it most likely holds every column to its end: M is
          * assembled right after it, and only if the counters then show a
          * column that moved on do the other launches of the chain (5 on empty
          * queues in FP64, 10 mixed: 21 and 33 us on the 256^2 and 371^2 grids)
          * and a second assembly follow (about 40 us).  Not with counters, whose launches are all listed. */
-        const bool alone = !a.work && straight_chain(ctx, routed, fp64_mode, ctx->plen_max) &&
+        const bool alone = !a.work && !routed.empty() && routed[0].group < kWave && straight_chain(ctx, routed, fp64_mode, ctx->plen_max) &&
                            4.0 * mean_first_list(ctx) <= routed[0].L.capSort;
         if ((rc = run_chain(ctx, a, bins, fbins, G, gwaves, mixed, fp64_mode, n, ctx->plen_max,
                             alone ? kFirstBin : kWholeChain)))
