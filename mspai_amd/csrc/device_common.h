@@ -166,7 +166,10 @@ struct BlockArgs {
     double* res;
     int* nsolve;
     int* status;
-    int* head;                // work counter of the persistent kernel
+    int* head;                // work counters of the LDS and the HBM kernel (head[0], head[2])
+    const int* queue;         // block columns of the HBM kernel (nullptr: all)
+    int* overflow;            // those the LDS kernel passes on
+    int* n_overflow;
     int* error;               // set when a column outgrew the working set
     char* scratch;            // per-wave working sets
 };
@@ -580,6 +583,59 @@ struct Group {
     }
     static __device__ __forceinline__ unsigned long long lanes_below() { return (1ull << lane()) - 1ull; }
 };
+
+/* Row-group layout for 64-lane groups: lane l = 16 c + q holds rows q,
+ * q + 16, q + 32, q + 48 (t = 0..3) of the columns j = c + 4 s (slot s =
+ * 0..7); the right-hand side is column 32 (c = 0, slot 8).  The dot product
+ * of a column adds its four rows in the lane first -- (p_t0 + p_t2) +
+ * (p_t1 + p_t3) are the xor-32 and xor-16 steps of the 64-lane order -- then
+ * the xor-8..1 steps run as DPP inside the 16-lane row, so every row group
+ * reduces its own column and no broadcast of the sums is needed.  The
+ * Householder vector of step i lives in row group i mod 4 and is copied to
+ * the other three with lane swaps. */
+
+/* value X of row group `src` (0..3) in every row group (same q) */
+__device__ __forceinline__ unsigned rowgroup_bcast(unsigned x, int src)
+{
+    auto a = __builtin_amdgcn_permlane16_swap(x, x, false, false);  // a[0]: rows 0,0,2,2; a[1]: 1,1,3,3
+    const unsigned z = (src & 1) ? a[1] : a[0];
+    auto b = __builtin_amdgcn_permlane32_swap(z, z, false, false);  // b[0]: z rows 0,1,0,1; b[1]: 2,3,2,3
+    return (src & 2) ? b[1] : b[0];
+}
+__device__ __forceinline__ double rowgroup_bcast(double x, int src)
+{
+    const long long v = __double_as_longlong(x);
+    const unsigned lo = rowgroup_bcast((unsigned)v, src), hi = rowgroup_bcast((unsigned)(v >> 32), src);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+/* value X of row group SRC (compile time) in row group 0 */
+template <int SRC>
+__device__ __forceinline__ unsigned rowgroup_to0(unsigned x)
+{
+    if (SRC == 0) return x;
+    if (SRC == 1) return __builtin_amdgcn_permlane16_swap(x, x, false, false)[1];
+    if (SRC == 2) return __builtin_amdgcn_permlane32_swap(x, x, false, false)[1];
+    const unsigned y = __builtin_amdgcn_permlane16_swap(x, x, false, false)[1];
+    return __builtin_amdgcn_permlane32_swap(y, y, false, false)[1];
+}
+template <int SRC>
+__device__ __forceinline__ double rowgroup_to0(double x)
+{
+    const long long v = __double_as_longlong(x);
+    const unsigned lo = rowgroup_to0<SRC>((unsigned)v), hi = rowgroup_to0<SRC>((unsigned)(v >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+/* the four in-lane rows, then xor 8..1 inside the 16-lane row */
+__device__ __forceinline__ double rowgroup_sum(const double (&p)[4])
+{
+    using Gr = Group<64>;
+    double v = (p[0] + p[2]) + (p[1] + p[3]);
+    v = Gr::sum_step<8>(v);
+    v = Gr::sum_step<4>(v);
+    v = Gr::sum_step<2>(v);
+    v = Gr::sum_step<1>(v);
+    return v;
+}
 
 /* Backwards-compatible whole-wave helpers. */
 __device__ __forceinline__ double wave_sum_fixed(double p) { return Group<64>::sum_fixed(p); }

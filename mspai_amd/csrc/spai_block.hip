@@ -110,7 +110,14 @@ __device__ __forceinline__ int sorted_union(const int* ptr, const int* ind, cons
         }
         int incl = W::scan_incl(len);
         int excl = incl - len;
-        for (int e = 0; e < len; ++e) buf[off + excl + e] = ind[e0 + e];
+        for (int e = 0; e < len; e += 8) {  // eight loads in flight
+            int v[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] = e + q < len ? ind[e0 + e + q] : 0;
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                if (e + q < len) buf[off + excl + e + q] = v[q];
+        }
         off += W::bcast_last(incl);
     }
     __syncthreads();
@@ -535,14 +542,427 @@ __device__ bool block_column(const BlockArgs& a, const BlockLayout& L, const Blk
     return true;
 }
 
+/* ---- block columns in LDS: |I| <= 64 and |J| <= 24 scalars, blocks to 4x4 ----
+ *
+ * Almost every block column stays in these sizes (of the 65,536 on the 256^2
+ * grid of three fields: FIG_SHARE).  With the working set in HBM each pass over
+ * A(I,J), the residual or the scores waited for memory, the blocks of J were
+ * gathered one column of A after another, and the register QR took four lane
+ * moves per dot product.  Here the working set is 18 KB of LDS (9 waves per
+ * CU), all blocks of J are gathered together, one per lane, the QR runs in the
+ * row-group layout (in-lane sums, the right-hand sides one per row group), and
+ * a candidate's numerator stays in registers.  FIG_BLOCK.  Bound by the latency
+ * of those chains.  A column that outgrows it, or whose scores tie across the
+ * cut, starts afresh in the HBM kernel: the same bits. */
+constexpr int kLdsRows = 64, kLdsCols = 24, kLdsB = 4, kLdsRaw = 512, kLdsU = 2 * kWave;
+
+struct BlkLds {
+    union {
+        double A[kLdsCols * kLdsRows];  // A(I,J), column-major: from the gather to the residual
+        int raw[kLdsRaw];               // index lists before sorting
+    };
+    double r[kLdsB * kLdsRows];
+    double x[kLdsB * kLdsCols];
+    int cand[kLdsU];
+    int J[kLdsCols], I[kLdsRows];  // blocks of at least one scalar each
+    int fr[kLdsRows + 1], fc[kLdsCols + 1];
+    int segs[kLdsCols], segoff[kLdsCols + 1];
+    int sel[kLdsCols];
+};
+
+/* Lane k of every row of 16 lanes, k a constant after unrolling. */
+template <int K = 0>
+__device__ __forceinline__ double row_lane(double v, int k)
+{
+    if constexpr (K >= 16) {
+        return 0.0;
+    } else {
+        if (k == K) return Group<16>::lane_bcast<K>(v);
+        return row_lane<K + 1>(v, k);
+    }
+}
+
+/* Approximative_Solution (block) in the row-group layout (lane 16 c + q: rows
+ * q + 16 t of the columns c + 4 s); right-hand side c, the identity's column
+ * at row e0 + c (none when e0 < 0), in slot NS of row group c.  Solution, or
+ * what block_solve_regs leaves for a degenerate R, in w.x; status bits. */
+__device__ __forceinline__ int block_solve_rows(BlkLds& w, int m, int n, int bk, int e0)
+{
+    constexpr int NS = kLdsCols / 4;
+    const int lane = W::lane();
+    const int c = lane >> 4, q = lane & 15;
+    double a[NS + 1][4];
+#pragma unroll
+    for (int sl = 0; sl < NS; ++sl)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int j = c + 4 * sl;
+            a[sl][t] = j < n ? w.A[j * kLdsRows + q + 16 * t] : 0.0;
+        }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) a[NS][t] = (c < bk && e0 >= 0 && q + 16 * t == e0 + c) ? 1.0 : 0.0;
+    const int k = m < n ? m : n;
+    bool zero_diag = false;
+#pragma unroll
+    for (int si = 0; si < NS; ++si) {
+        if (4 * si >= k) break;
+#pragma unroll 1
+        for (int ci = 0; ci < 4; ++ci) {
+            const int i = 4 * si + ci;
+            if (i >= k) break;
+            double p[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) p[t] = q + 16 * t > i ? __fma_rn(a[si][t], a[si][t], 0.0) : 0.0;
+            const double xn2 = W::lane_value(rowgroup_sum(p), 16 * ci);
+            const double alpha = W::lane_value((i >> 4) ? a[si][1] : a[si][0], 16 * ci + (i & 15));
+            double rii = alpha;
+            if (i + 1 < m && xn2 != 0.0) {
+                const double nrm = sqrt(__fma_rn(alpha, alpha, xn2));
+                const double beta = -copysign(nrm, alpha);
+                const double tau = (beta - alpha) / beta;
+                const double scal = 1.0 / (alpha - beta);
+                rii = beta;
+                double v[4];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const int r = q + 16 * t;
+                    const double vl = r > i ? a[si][t] * scal : (r == i ? 1.0 : 0.0);
+                    v[t] = rowgroup_bcast(vl, ci);
+                    if (c == ci && r == i) a[si][t] = beta;
+                    else if (c == ci && r > i) a[si][t] = vl;
+                }
+                const double mt = -tau;
+#pragma unroll
+                for (int sl = si; sl <= NS; ++sl) {
+                    if ((4 * sl + 3 > i && 4 * sl < n) || sl == NS) {
+                        const int j = c + 4 * sl;
+                        const bool live = sl == NS ? c < bk : (j > i && j < n);
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) p[t] = q + 16 * t >= i ? __fma_rn(v[t], a[sl][t], 0.0) : 0.0;
+                        const double tw = mt * rowgroup_sum(p);
+#pragma unroll
+                        for (int t = 0; t < 4; ++t)
+                            if (live && q + 16 * t >= i) a[sl][t] = __fma_rn(v[t], tw, a[sl][t]);
+                    }
+                }
+            }
+            zero_diag |= rii == 0.0;
+        }
+    }
+    int st = 0;
+    if (m < n) {
+        st = COL_UNDERDET;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) a[NS][t] = 0.0;
+    } else if (zero_diag) {
+        st = COL_SINGULAR;  // dtrtrs leaves Q^T E
+    } else {
+        /* dtrsm order, every right-hand side in its row group */
+#pragma unroll
+        for (int K = kLdsCols - 1; K >= 0; --K) {
+            if (K < n) {
+                const int sK = K >> 2, tK = K >> 4, qK = K & 15;
+                double xk = row_lane(a[NS][tK], qK);
+                const double rkk = W::lane_value(a[sK][tK], 16 * (K & 3) + qK);
+                const bool nz = xk != 0.0;
+                xk = xk / rkk;
+#pragma unroll
+                for (int t = 0; t <= tK; ++t) {
+                    const int r = q + 16 * t;
+                    const double u = __fma_rn(-xk, rowgroup_bcast(a[sK][t], K & 3), a[NS][t]);
+                    a[NS][t] = nz ? (r == K ? xk : (r < K ? u : a[NS][t])) : a[NS][t];
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; 16 * t < kLdsCols; ++t)
+        if (c < bk && q + 16 * t < n) w.x[c * n + q + 16 * t] = a[NS][t];
+    __syncthreads();
+    return st;
+}
+
+/* Augment_Sparsity_Block as augment_block; kBlkOverflow also when the scores
+ * tie across the cut. */
+__device__ __forceinline__ int augment_lds(const BlockArgs& a, BlkLds& w, int col, int bk, int mi, int nj, double rn,
+                                           int* st)
+{
+    const int lane = W::lane();
+    const int p = lower_bound_i(w.I, mi, col);
+    const bool col_in = p < mi && w.I[p] == col;
+    const int nu = sorted_union(a.rp_ptr, a.rp_ind, w.I, mi, col_in ? -1 : col, w.raw, kLdsRaw, w.raw);
+    if (nu == kBlkOverflow) return kBlkOverflow;
+    int c = 0;
+    for (int base = 0; base < nu; base += kWave) {
+        const int t = base + lane;
+        const int u = t < nu ? w.raw[t] : 0;
+        bool keep = false;
+        if (t < nu) {
+            const int q = lower_bound_i(w.J, nj, u);
+            keep = !(q < nj && w.J[q] == u);
+        }
+        const unsigned long long mask = W::ballot(keep);
+        if (c + __popcll(mask) > kLdsU) return kBlkOverflow;
+        if (keep) w.cand[c + __popcll(mask & W::lanes_below())] = u;
+        c += __popcll(mask);
+    }
+    __syncthreads();
+    if (c == 0) return -1;
+    /* one candidate per lane, two rounds at most; the scores stay in registers */
+    double rho[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        rho[u] = INFINITY;
+        const int t = lane + kWave * u;
+        if (t < c) {
+            const int j = w.cand[t], bj = a.bsize[j];
+            const double* inv = a.sqinv + a.sqoff[j];
+            double N[kLdsB * kLdsB];
+#pragma unroll
+            for (int e = 0; e < kLdsB * kLdsB; ++e) N[e] = 0.0;
+            const int e1 = a.colptr[j + 1];
+            for (int e = a.colptr[j]; e < e1; ++e) {
+                const int ib = a.rowind[e];
+                const int at = lower_bound_i(w.I, mi, ib);
+                if (at >= mi || w.I[at] != ib) continue;
+                const int r0 = w.fr[at], h = w.fr[at + 1] - r0;
+                const double* const av = a.val + a.voff[e];
+                double v[kLdsB * kLdsB];  // column ii of the block at ii * kLdsB
+#pragma unroll
+                for (int ii = 0; ii < kLdsB; ++ii)
+#pragma unroll
+                    for (int tt = 0; tt < kLdsB; ++tt)
+                        v[ii * kLdsB + tt] = (ii < bj && tt < h) ? av[ii * h + tt] : 0.0;
+#pragma unroll
+                for (int qq = 0; qq < kLdsB; ++qq)
+                    if (qq < bk) {
+                        double rv[kLdsB];
+#pragma unroll
+                        for (int tt = 0; tt < kLdsB; ++tt) rv[tt] = tt < h ? w.r[qq * kLdsRows + r0 + tt] : 0.0;
+#pragma unroll
+                        for (int ii = 0; ii < kLdsB; ++ii) {
+                            double s = 0.0;
+#pragma unroll
+                            for (int tt = 0; tt < kLdsB; ++tt)
+                                if (tt < h) s = __fma_rn(v[ii * kLdsB + tt], rv[tt], s);
+                            if (ii < bj) N[qq * kLdsB + ii] = __dadd_rn(N[qq * kLdsB + ii], s);
+                        }
+                    }
+            }
+            double iv[kLdsB * kLdsB];
+#pragma unroll
+            for (int kk = 0; kk < kLdsB; ++kk)
+#pragma unroll
+                for (int ii = 0; ii < kLdsB; ++ii)
+                    iv[kk * kLdsB + ii] = (kk < bj && ii < bj) ? inv[kk * bj + ii] : 0.0;
+            double term = 0.0;
+#pragma unroll
+            for (int qq = 0; qq < kLdsB; ++qq)
+#pragma unroll
+                for (int ii = 0; ii < kLdsB; ++ii)
+                    if (qq < bk && ii < bj) {
+                        double s = 0.0;
+#pragma unroll
+                        for (int kk = 0; kk < kLdsB; ++kk)
+                            if (kk < bj) s = __fma_rn(iv[kk * kLdsB + ii], N[qq * kLdsB + kk], s);
+                        term = __dadd_rn(term, __dmul_rn(s, N[qq * kLdsB + ii]));
+                    }
+            rho[u] = sqrt(__dsub_rn(__dmul_rn(rn, rn), term));
+        }
+    }
+    double mean = 0.0;
+    for (int t = 0; t < c; ++t) mean = __dadd_rn(mean, W::lane_value(t < kWave ? rho[0] : rho[1], t & (kWave - 1)));
+    if (a.use_mean) mean = __ddiv_rn(mean, (double)c);
+    if (isnan(mean)) {
+        *st |= COL_NAN_RHO;
+        return nj;
+    }
+    const bool in[2] = {lane < c, lane + kWave < c};
+    int qn = 0;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) qn += __popcll(W::ballot(in[u] && rho[u] <= mean));
+    const int sneed = a.maxnew < qn ? a.maxnew : qn;
+    if (sneed <= 0) return nj;
+    if (nj + sneed > kLdsCols) return kBlkOverflow;
+    /* the sneed-th smallest score and the number of scores below it */
+    double prev = -1.0, vstar = 0.0;
+    int below = 0, ties = 0;
+    for (int it = 0; it < c; ++it) {
+        double v = INFINITY;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+            if (in[u] && rho[u] > prev) v = fmin(v, rho[u]);
+        v = W::min(v);
+        int cnt = 0;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) cnt += __popcll(W::ballot(in[u] && rho[u] == v));
+        if (below + cnt >= sneed || cnt == 0) {
+            vstar = v;
+            ties = cnt;
+            break;
+        }
+        below += cnt;
+        prev = v;
+    }
+    if (sneed - below != ties) return kBlkOverflow;  // std::sort's order decides
+    int ns = 0;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const bool keep = in[u] && rho[u] <= vstar;
+        const unsigned long long mask = W::ballot(keep);
+        if (keep) w.sel[ns + __popcll(mask & W::lanes_below())] = w.cand[lane + kWave * u];
+        ns += __popcll(mask);
+    }
+    __syncthreads();
+    if (lane == 0) {
+        int i = nj - 1, t = sneed - 1, o = nj + sneed - 1;
+        while (t >= 0) {
+            if (i >= 0 && w.J[i] > w.sel[t]) w.J[o--] = w.J[i--];
+            else w.J[o--] = w.sel[t--];
+        }
+    }
+    __syncthreads();
+    return nj + sneed;
+}
+
+/* One block column; false when it goes to the HBM kernel. */
+__device__ __forceinline__ bool block_column_lds(const BlockArgs& a, BlkLds& w, int col)
+{
+    const int lane = W::lane();
+    const int bk = a.bsize[col];
+    const double eps = a.epsilon * sqrt((double)bk);  // adjust_epsilon
+    const int p0 = a.p_ptr[col];
+    int nj = a.p_ptr[col + 1] - p0;
+    if (nj > kLdsCols) return false;
+    if (lane < nj) w.J[lane] = a.p_ind[p0 + lane];
+    __syncthreads();
+    int st = 0, solves = 0, n = 0;
+    double rn = 1.0e50;
+    for (int step = -1; step < a.ns; ++step) {
+        const int mi = sorted_union(a.colptr, a.rowind, w.J, nj, -1, w.raw, kLdsRaw, w.raw);
+        if (mi == kBlkOverflow || mi > kLdsRows) return false;
+        if (lane < mi) w.I[lane] = w.raw[lane];
+        __syncthreads();
+        const int m = prefix_sizes(a.bsize, w.I, mi, w.fr);
+        n = prefix_sizes(a.bsize, w.J, nj, w.fc);
+        if (m > kLdsRows || n > kLdsCols) return false;
+        for (int c = 0; c < n; ++c) w.A[c * kLdsRows + lane] = 0.0;
+        int start = 0, cnt = 0;
+        if (lane < nj) {
+            start = a.colptr[w.J[lane]];
+            cnt = a.colptr[w.J[lane] + 1] - start;
+        }
+        const int incl = W::scan_incl(cnt), total = W::bcast_last(incl);
+        if (lane < nj) {
+            w.segs[lane] = start;
+            w.segoff[lane] = incl - cnt;
+        }
+        __syncthreads();
+        /* one block of A(I,J) per lane */
+        for (int e = lane; e < total; e += kWave) {
+            int t = 0, hi = nj;
+            while (hi - t > 1) {
+                const int mid = (t + hi) >> 1;
+                if (w.segoff[mid] <= e) t = mid;
+                else hi = mid;
+            }
+            const int src = w.segs[t] + e - w.segoff[t];
+            const double* const blk = a.val + a.voff[src];
+            const int pos = lower_bound_i(w.I, mi, a.rowind[src]);
+            const int r0 = w.fr[pos], h = w.fr[pos + 1] - r0, c0 = w.fc[t], bj = w.fc[t + 1] - c0;
+            double v[kLdsB * kLdsB];
+#pragma unroll
+            for (int c = 0; c < kLdsB; ++c)
+#pragma unroll
+                for (int r = 0; r < kLdsB; ++r) v[c * kLdsB + r] = (c < bj && r < h) ? blk[c * h + r] : 0.0;
+#pragma unroll
+            for (int c = 0; c < kLdsB; ++c)
+#pragma unroll
+                for (int r = 0; r < kLdsB; ++r)
+                    if (c < bj && r < h) w.A[(c0 + c) * kLdsRows + r0 + r] = v[c * kLdsB + r];
+        }
+        __syncthreads();
+        /* E_k: the identity block at block row col's offset */
+        const int pk = lower_bound_i(w.I, mi, col);
+        const int e0 = pk < mi && w.I[pk] == col ? w.fr[pk] : -1;
+        if (e0 < 0) st |= COL_K_NOT_IN_I;
+        st |= block_solve_rows(w, m, n, bk, e0);
+        ++solves;
+        /* R = A(I,J) X - E, row `lane`, then the Frobenius norm in order */
+        double r[kLdsB];
+#pragma unroll
+        for (int q = 0; q < kLdsB; ++q) r[q] = -((e0 >= 0 && lane == e0 + q) ? 1.0 : 0.0);
+        for (int jj = 0; jj < n; ++jj) {
+            const double aij = w.A[jj * kLdsRows + lane];
+#pragma unroll
+            for (int q = 0; q < kLdsB; ++q)
+                if (q < bk) {
+                    const double xj = w.x[q * n + jj];
+                    const double t = __fma_rn(xj, aij, r[q]);
+                    r[q] = xj != 0.0 ? t : r[q];
+                }
+        }
+        double sum = 0.0;
+#pragma unroll
+        for (int q = 0; q < kLdsB; ++q)
+            if (q < bk) {
+                w.r[q * kLdsRows + lane] = r[q];
+                const double sq = __dmul_rn(r[q], r[q]);
+                for (int i = 0; i < m; ++i) sum = __dadd_rn(sum, W::lane_value(sq, i));
+            }
+        __syncthreads();
+        rn = sqrt(sum);
+        if (rn <= eps || step == a.ns - 1) break;
+        const int nn = augment_lds(a, w, col, bk, mi, nj, rn, &st);
+        if (nn == kBlkOverflow) return false;
+        if (nn < 0) break;
+        nj = nn;
+    }
+    const size_t ov = (size_t)col * a.capX;
+    for (int t = 0; t < nj; ++t) {
+        const int f = w.fc[t], bj = w.fc[t + 1] - f;
+        if (lane < bj * bk) {
+            const int q = lane / bj, jj = lane - q * bj;
+            a.m_val[ov + (size_t)f * bk + lane] = w.x[q * n + f + jj];
+        }
+    }
+    if (lane < nj) a.m_idx[(size_t)col * a.capJ + lane] = w.J[lane];
+    if (lane == 0) {
+        a.m_len[col] = nj;
+        a.res[col] = rn;
+        a.nsolve[col] = solves;
+        a.status[col] = st;
+    }
+    __syncthreads();
+    return true;
+}
+
+__global__ __launch_bounds__(64, 3) void block_lds_kernel(BlockArgs a)
+{
+    __shared__ BlkLds w;
+    constexpr int kChunk = 4;  // columns per draw from the queue
+    for (;;) {
+        int c = 0;
+        if (lane_id() == 0) c = atomicAdd(a.head, kChunk);
+        const int c0 = __builtin_amdgcn_readlane(c, 0);
+        if (c0 >= a.nb) break;
+        for (int col = c0; col < a.nb && col < c0 + kChunk; ++col) {
+            if (!block_column_lds(a, w, col) && lane_id() == 0) a.overflow[atomicAdd(a.n_overflow, 1)] = col;
+            __syncthreads();
+        }
+    }
+}
+
 __global__ __launch_bounds__(64, 4) void block_column_kernel(BlockArgs a, BlockLayout L)
 {
     BlkScratch s = blk_scratch(a.scratch + (size_t)blockIdx.x * L.per_wave, L);
+    const int count = a.queue ? *a.n_overflow : a.nb;
     for (;;) {
         int c = 0;
-        if (lane_id() == 0) c = atomicAdd(a.head, 1);
-        const int col = __builtin_amdgcn_readlane(c, 0);
-        if (col >= a.nb) break;
+        if (lane_id() == 0) c = atomicAdd(a.head + 2, 1);
+        c = __builtin_amdgcn_readlane(c, 0);
+        if (c >= count) break;
+        const int col = a.queue ? a.queue[c] : c;
         if (!block_column(a, L, s, col) && lane_id() == 0) {
             a.m_len[col] = 0;  // the scalar conversion reads only what was written
             atomicOr(a.error, 1);
@@ -688,6 +1108,14 @@ void launch_block_sq_inverse(const BlockArgs& a, double* tmp, hipStream_t stream
 {
     if (a.nb <= 0) return;
     hipLaunchKernelGGL(block_sq_inverse_kernel, dim3((a.nb + 63) / 64), dim3(64), 0, stream, a, tmp);
+}
+
+bool launch_block_lds(const BlockArgs& a, int maxbs, int num_cu, hipStream_t stream)
+{
+    if (maxbs > kLdsB) return false;
+    const int per_cu = (160 << 10) / (int)sizeof(BlkLds);
+    hipLaunchKernelGGL(block_lds_kernel, dim3(num_cu * per_cu), dim3(kWave), 0, stream, a);
+    return true;
 }
 
 void launch_block_columns(const BlockArgs& a, const BlockLayout& L, int nwaves, hipStream_t stream)

@@ -81,7 +81,10 @@ void launch_line_dot(int nlines, const int* ptr, const int* ind, const double* v
 void launch_block_values(const BlockArgs& a, const DevCsc& A, const int* bmap, double* bval, hipStream_t stream);
 /* (A_j^T A_j)^-1 of every block column into a.sqinv (tmp: sum bsize^2 doubles). */
 void launch_block_sq_inverse(const BlockArgs& a, double* tmp, hipStream_t stream);
-/* Persistent block-column kernel on nwaves waves, L.per_wave bytes each at a.scratch. */
+/* Block columns with the working set in LDS; those it cannot hold go to
+ * a.overflow.  False, nothing launched: blocks wider than it takes. */
+bool launch_block_lds(const BlockArgs& a, int maxbs, int num_cu, hipStream_t stream);
+/* Persistent block-column kernel (a.queue, or all block columns) on nwaves waves, L.per_wave bytes each at a.scratch. */
 void launch_block_columns(const BlockArgs& a, const BlockLayout& L, int nwaves, hipStream_t stream);
 /* Scalar_Matrix: per-scalar-column nonzero counts, then the CSC fill. */
 void launch_block_scalar_count(const BlockArgs& a, int* counts, hipStream_t stream);
