@@ -2596,19 +2596,19 @@ static int build_block(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* stat
     a.nsolve = ctx->d_nsolve;
     a.status = ctx->d_status;
     a.head = ctx->d_counter + 56;
-    a.error = ctx->d_counter + 57;
+    a.error = ctx->d_counter + 59;
     a.overflow = ctx->d_queues;
-    a.n_overflow = ctx->d_counter + 59;
+    a.n_overflow = ctx->d_counter + 60;
     a.scratch = ctx->d_bscratch;
 
     HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
-    HIPCHK(hipMemsetAsync(ctx->d_counter + 56, 0, 4 * sizeof(int), ctx->stream));
+    HIPCHK(hipMemsetAsync(ctx->d_counter + 56, 0, 6 * sizeof(int), ctx->stream));
     ctx->last_counters = false;  // the block kernel keeps no work counters
     ctx->nlaunch = 0;            // nor a per-launch profile
     ctx->lwork_valid = false;
     if (ns > 0) launch_block_sq_inverse(a, ctx->d_sqtmp, ctx->stream);
     HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
-    if (launch_block_lds(a, mb, ctx->num_cu, ctx->stream)) a.queue = ctx->d_queues;
+    if (launch_block_lds(a, mb, ctx->num_cu, ctx->stream)) a.queue = ctx->d_queues + nb;
     launch_block_columns(a, L, (int)nwaves, ctx->stream);
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(ctx->ev[2], ctx->stream));
@@ -2623,7 +2623,7 @@ static int build_block(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* stat
     HIPCHK(hipEventRecord(ctx->ev[3], ctx->stream));
     if ((rc = fetch_counters(ctx))) return rc;
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    if (ctx->h_counter[57])
+    if (ctx->h_counter[59])
         return fail(ctx, MSPAI_ERR_CAPACITY, "block build: a block column outgrew its working set");
     const int last = ctx->h_counter[63];
     ctx->nnzM = last;

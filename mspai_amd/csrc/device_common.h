@@ -166,10 +166,10 @@ struct BlockArgs {
     double* res;
     int* nsolve;
     int* status;
-    int* head;                // work counters of the LDS and the HBM kernel (head[0], head[2])
+    int* head;                // work counters of the two LDS stages and of the HBM kernel
     const int* queue;         // block columns of the HBM kernel (nullptr: all)
-    int* overflow;            // those the LDS kernel passes on
-    int* n_overflow;
+    int* overflow;            // those the LDS stages pass on: nb entries for each
+    int* n_overflow;          // their numbers
     int* error;               // set when a column outgrew the working set
     char* scratch;            // per-wave working sets
 };

@@ -554,9 +554,15 @@ __device__ bool block_column(const BlockArgs& a, const BlockLayout& L, const Blk
  * a candidate's numerator stays in registers.  FIG_BLOCK.  Bound by the latency
  * of those chains.  A column that outgrows it, or whose scores tie across the
  * cut, starts afresh in the HBM kernel: the same bits. */
-constexpr int kLdsRows = 64, kLdsCols = 24, kLdsB = 4, kLdsRaw = 512, kLdsU = 2 * kWave;
+constexpr int kLdsB = 4, kLdsRaw = 512, kLdsU = 2 * kWave;
 
+/* Working set of |I| <= kLdsRows (64 or 128), |J| <= kLdsCols scalars. */
+template <int ROWS, int COLS>
 struct BlkLds {
+    static constexpr int kLdsRows = ROWS, kLdsCols = COLS;
+    static constexpr int RT = ROWS / 16;   // rows per lane of the row-group layout
+    static constexpr int kOwn = ROWS / kWave;  // rows per lane in row order
+    static_assert(RT == 4 || RT == 8, "rows");
     union {
         double A[kLdsCols * kLdsRows];  // A(I,J), column-major: from the gather to the residual
         int raw[kLdsRaw];               // index lists before sorting
@@ -586,21 +592,32 @@ __device__ __forceinline__ double row_lane(double v, int k)
  * q + 16 t of the columns c + 4 s); right-hand side c, the identity's column
  * at row e0 + c (none when e0 < 0), in slot NS of row group c.  Solution, or
  * what block_solve_regs leaves for a degenerate R, in w.x; status bits. */
-__device__ __forceinline__ int block_solve_rows(BlkLds& w, int m, int n, int bk, int e0)
+template <class B>
+__device__ __forceinline__ int block_solve_rows(B& w, int m, int n, int bk, int e0)
 {
-    constexpr int NS = kLdsCols / 4;
+    constexpr int kLdsRows = B::kLdsRows, kLdsCols = B::kLdsCols, NS = kLdsCols / 4, RT = B::RT;
     const int lane = W::lane();
     const int c = lane >> 4, q = lane & 15;
-    double a[NS + 1][4];
+    double a[NS + 1][RT];
+    /* the 64-lane order: row r + 64 continues the chain of row r */
+    auto sum = [&](auto term) {
+        double p[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            p[t] = term(t, 0.0);
+            if constexpr (RT == 8) p[t] = term(t + 4, p[t]);
+        }
+        return rowgroup_sum(p);
+    };
 #pragma unroll
     for (int sl = 0; sl < NS; ++sl)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+        for (int t = 0; t < RT; ++t) {
             const int j = c + 4 * sl;
             a[sl][t] = j < n ? w.A[j * kLdsRows + q + 16 * t] : 0.0;
         }
 #pragma unroll
-    for (int t = 0; t < 4; ++t) a[NS][t] = (c < bk && e0 >= 0 && q + 16 * t == e0 + c) ? 1.0 : 0.0;
+    for (int t = 0; t < RT; ++t) a[NS][t] = (c < bk && e0 >= 0 && q + 16 * t == e0 + c) ? 1.0 : 0.0;
     const int k = m < n ? m : n;
     bool zero_diag = false;
 #pragma unroll
@@ -610,11 +627,12 @@ __device__ __forceinline__ int block_solve_rows(BlkLds& w, int m, int n, int bk,
         for (int ci = 0; ci < 4; ++ci) {
             const int i = 4 * si + ci;
             if (i >= k) break;
-            double p[4];
+            const double xn2 = W::lane_value(
+                sum([&](int t, double s0) { return q + 16 * t > i ? __fma_rn(a[si][t], a[si][t], s0) : s0; }), 16 * ci);
+            double aii = a[si][0];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) p[t] = q + 16 * t > i ? __fma_rn(a[si][t], a[si][t], 0.0) : 0.0;
-            const double xn2 = W::lane_value(rowgroup_sum(p), 16 * ci);
-            const double alpha = W::lane_value((i >> 4) ? a[si][1] : a[si][0], 16 * ci + (i & 15));
+            for (int t = 1; 16 * t < kLdsCols; ++t) aii = (i >> 4) == t ? a[si][t] : aii;
+            const double alpha = W::lane_value(aii, 16 * ci + (i & 15));
             double rii = alpha;
             if (i + 1 < m && xn2 != 0.0) {
                 const double nrm = sqrt(__fma_rn(alpha, alpha, xn2));
@@ -622,9 +640,9 @@ __device__ __forceinline__ int block_solve_rows(BlkLds& w, int m, int n, int bk,
                 const double tau = (beta - alpha) / beta;
                 const double scal = 1.0 / (alpha - beta);
                 rii = beta;
-                double v[4];
+                double v[RT];
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
+                for (int t = 0; t < RT; ++t) {
                     const int r = q + 16 * t;
                     const double vl = r > i ? a[si][t] * scal : (r == i ? 1.0 : 0.0);
                     v[t] = rowgroup_bcast(vl, ci);
@@ -637,11 +655,11 @@ __device__ __forceinline__ int block_solve_rows(BlkLds& w, int m, int n, int bk,
                     if ((4 * sl + 3 > i && 4 * sl < n) || sl == NS) {
                         const int j = c + 4 * sl;
                         const bool live = sl == NS ? c < bk : (j > i && j < n);
+                        const double tw = mt * sum([&](int t, double s0) {
+                            return q + 16 * t >= i ? __fma_rn(v[t], a[sl][t], s0) : s0;
+                        });
 #pragma unroll
-                        for (int t = 0; t < 4; ++t) p[t] = q + 16 * t >= i ? __fma_rn(v[t], a[sl][t], 0.0) : 0.0;
-                        const double tw = mt * rowgroup_sum(p);
-#pragma unroll
-                        for (int t = 0; t < 4; ++t)
+                        for (int t = 0; t < RT; ++t)
                             if (live && q + 16 * t >= i) a[sl][t] = __fma_rn(v[t], tw, a[sl][t]);
                     }
                 }
@@ -653,7 +671,7 @@ __device__ __forceinline__ int block_solve_rows(BlkLds& w, int m, int n, int bk,
     if (m < n) {
         st = COL_UNDERDET;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) a[NS][t] = 0.0;
+        for (int t = 0; t < RT; ++t) a[NS][t] = 0.0;
     } else if (zero_diag) {
         st = COL_SINGULAR;  // dtrtrs leaves Q^T E
     } else {
@@ -684,9 +702,11 @@ __device__ __forceinline__ int block_solve_rows(BlkLds& w, int m, int n, int bk,
 
 /* Augment_Sparsity_Block as augment_block; kBlkOverflow also when the scores
  * tie across the cut. */
-__device__ __forceinline__ int augment_lds(const BlockArgs& a, BlkLds& w, int col, int bk, int mi, int nj, double rn,
+template <class B>
+__device__ __forceinline__ int augment_lds(const BlockArgs& a, B& w, int col, int bk, int mi, int nj, double rn,
                                            int* st)
 {
+    constexpr int kLdsRows = B::kLdsRows, kLdsCols = B::kLdsCols;
     const int lane = W::lane();
     const int p = lower_bound_i(w.I, mi, col);
     const bool col_in = p < mi && w.I[p] == col;
@@ -720,13 +740,28 @@ __device__ __forceinline__ int augment_lds(const BlockArgs& a, BlkLds& w, int co
             double N[kLdsB * kLdsB];
 #pragma unroll
             for (int e = 0; e < kLdsB * kLdsB; ++e) N[e] = 0.0;
-            const int e1 = a.colptr[j + 1];
-            for (int e = a.colptr[j]; e < e1; ++e) {
-                const int ib = a.rowind[e];
-                const int at = lower_bound_i(w.I, mi, ib);
-                if (at >= mi || w.I[at] != ib) continue;
-                const int r0 = w.fr[at], h = w.fr[at + 1] - r0;
-                const double* const av = a.val + a.voff[e];
+            const int e0 = a.colptr[j], e1 = a.colptr[j + 1];
+            constexpr int kR = 8;  // entries whose rows and offsets load together
+            for (int eb = e0; eb < e1; eb += kR) {
+            int at[kR];
+            long long voff[kR];
+#pragma unroll
+            for (int x = 0; x < kR; ++x) {
+                at[x] = eb + x < e1 ? a.rowind[eb + x] : -1;
+                voff[x] = eb + x < e1 ? a.voff[eb + x] : 0;
+            }
+#pragma unroll
+            for (int x = 0; x < kR; ++x) {
+                const int ib = at[x];
+                if (ib < 0) continue;
+                at[x] = lower_bound_i(w.I, mi, ib);
+                if (at[x] >= mi || w.I[at[x]] != ib) at[x] = -1;
+            }
+#pragma unroll
+            for (int x = 0; x < kR; ++x) {
+                if (at[x] < 0) continue;
+                const int r0 = w.fr[at[x]], h = w.fr[at[x] + 1] - r0;
+                const double* const av = a.val + voff[x];
                 double v[kLdsB * kLdsB];  // column ii of the block at ii * kLdsB
 #pragma unroll
                 for (int ii = 0; ii < kLdsB; ++ii)
@@ -748,6 +783,7 @@ __device__ __forceinline__ int augment_lds(const BlockArgs& a, BlkLds& w, int co
                             if (ii < bj) N[qq * kLdsB + ii] = __dadd_rn(N[qq * kLdsB + ii], s);
                         }
                     }
+            }
             }
             double iv[kLdsB * kLdsB];
 #pragma unroll
@@ -826,8 +862,10 @@ __device__ __forceinline__ int augment_lds(const BlockArgs& a, BlkLds& w, int co
 }
 
 /* One block column; false when it goes to the HBM kernel. */
-__device__ __forceinline__ bool block_column_lds(const BlockArgs& a, BlkLds& w, int col)
+template <class B>
+__device__ __forceinline__ bool block_column_lds(const BlockArgs& a, B& w, int col)
 {
+    constexpr int kLdsRows = B::kLdsRows, kLdsCols = B::kLdsCols, kOwn = B::kOwn;
     const int lane = W::lane();
     const int bk = a.bsize[col];
     const double eps = a.epsilon * sqrt((double)bk);  // adjust_epsilon
@@ -841,12 +879,12 @@ __device__ __forceinline__ bool block_column_lds(const BlockArgs& a, BlkLds& w, 
     for (int step = -1; step < a.ns; ++step) {
         const int mi = sorted_union(a.colptr, a.rowind, w.J, nj, -1, w.raw, kLdsRaw, w.raw);
         if (mi == kBlkOverflow || mi > kLdsRows) return false;
-        if (lane < mi) w.I[lane] = w.raw[lane];
+        for (int t = lane; t < mi; t += kWave) w.I[t] = w.raw[t];
         __syncthreads();
         const int m = prefix_sizes(a.bsize, w.I, mi, w.fr);
         n = prefix_sizes(a.bsize, w.J, nj, w.fc);
         if (m > kLdsRows || n > kLdsCols) return false;
-        for (int c = 0; c < n; ++c) w.A[c * kLdsRows + lane] = 0.0;
+        for (int c = lane; c < n * kLdsRows; c += kWave) w.A[c] = 0.0;
         int start = 0, cnt = 0;
         if (lane < nj) {
             start = a.colptr[w.J[lane]];
@@ -888,27 +926,35 @@ __device__ __forceinline__ bool block_column_lds(const BlockArgs& a, BlkLds& w, 
         if (e0 < 0) st |= COL_K_NOT_IN_I;
         st |= block_solve_rows(w, m, n, bk, e0);
         ++solves;
-        /* R = A(I,J) X - E, row `lane`, then the Frobenius norm in order */
-        double r[kLdsB];
+        /* R = A(I,J) X - E, rows lane and lane + 64, then the Frobenius norm in order */
+        double r[kOwn][kLdsB];
 #pragma unroll
-        for (int q = 0; q < kLdsB; ++q) r[q] = -((e0 >= 0 && lane == e0 + q) ? 1.0 : 0.0);
+        for (int u = 0; u < kOwn; ++u)
+#pragma unroll
+            for (int q = 0; q < kLdsB; ++q) r[u][q] = -((e0 >= 0 && lane + kWave * u == e0 + q) ? 1.0 : 0.0);
         for (int jj = 0; jj < n; ++jj) {
-            const double aij = w.A[jj * kLdsRows + lane];
 #pragma unroll
-            for (int q = 0; q < kLdsB; ++q)
-                if (q < bk) {
-                    const double xj = w.x[q * n + jj];
-                    const double t = __fma_rn(xj, aij, r[q]);
-                    r[q] = xj != 0.0 ? t : r[q];
-                }
+            for (int u = 0; u < kOwn; ++u) {
+                const double aij = w.A[jj * kLdsRows + lane + kWave * u];
+#pragma unroll
+                for (int q = 0; q < kLdsB; ++q)
+                    if (q < bk) {
+                        const double xj = w.x[q * n + jj];
+                        const double t = __fma_rn(xj, aij, r[u][q]);
+                        r[u][q] = xj != 0.0 ? t : r[u][q];
+                    }
+            }
         }
         double sum = 0.0;
 #pragma unroll
         for (int q = 0; q < kLdsB; ++q)
             if (q < bk) {
-                w.r[q * kLdsRows + lane] = r[q];
-                const double sq = __dmul_rn(r[q], r[q]);
-                for (int i = 0; i < m; ++i) sum = __dadd_rn(sum, W::lane_value(sq, i));
+#pragma unroll
+                for (int u = 0; u < kOwn; ++u) {
+                    w.r[q * kLdsRows + lane + kWave * u] = r[u][q];
+                    const double sq = __dmul_rn(r[u][q], r[u][q]);
+                    for (int i = 0; i < min(m - kWave * u, kWave); ++i) sum = __dadd_rn(sum, W::lane_value(sq, i));
+                }
             }
         __syncthreads();
         rn = sqrt(sum);
@@ -937,17 +983,25 @@ __device__ __forceinline__ bool block_column_lds(const BlockArgs& a, BlkLds& w, 
     return true;
 }
 
-__global__ __launch_bounds__(64, 3) void block_lds_kernel(BlockArgs a)
+/* Block columns of a.queue (all without one); kStage 0, 1: the stage's work
+ * counter, queue length and overflow queue. */
+template <int ROWS, int COLS, int kStage>
+__global__ __launch_bounds__(64, kStage == 0 ? 3 : 1) void block_lds_kernel(BlockArgs a)
 {
-    __shared__ BlkLds w;
-    constexpr int kChunk = 4;  // columns per draw from the queue
+    __shared__ BlkLds<ROWS, COLS> w;
+    constexpr int kChunk = kStage == 0 ? 4 : 1;  // columns per draw from the queue
+    int* const head = a.head + kStage;
+    const int* const queue = kStage == 0 ? nullptr : a.overflow;
+    int* const out = a.overflow + (size_t)kStage * a.nb;
+    const int count = queue ? a.n_overflow[0] : a.nb;
     for (;;) {
         int c = 0;
-        if (lane_id() == 0) c = atomicAdd(a.head, kChunk);
+        if (lane_id() == 0) c = atomicAdd(head, kChunk);
         const int c0 = __builtin_amdgcn_readlane(c, 0);
-        if (c0 >= a.nb) break;
-        for (int col = c0; col < a.nb && col < c0 + kChunk; ++col) {
-            if (!block_column_lds(a, w, col) && lane_id() == 0) a.overflow[atomicAdd(a.n_overflow, 1)] = col;
+        if (c0 >= count) break;
+        for (int c1 = c0; c1 < count && c1 < c0 + kChunk; ++c1) {
+            const int col = queue ? queue[c1] : c1;
+            if (!block_column_lds(a, w, col) && lane_id() == 0) out[atomicAdd(a.n_overflow + kStage, 1)] = col;
             __syncthreads();
         }
     }
@@ -956,7 +1010,7 @@ __global__ __launch_bounds__(64, 3) void block_lds_kernel(BlockArgs a)
 __global__ __launch_bounds__(64, 4) void block_column_kernel(BlockArgs a, BlockLayout L)
 {
     BlkScratch s = blk_scratch(a.scratch + (size_t)blockIdx.x * L.per_wave, L);
-    const int count = a.queue ? *a.n_overflow : a.nb;
+    const int count = a.queue ? a.n_overflow[1] : a.nb;
     for (;;) {
         int c = 0;
         if (lane_id() == 0) c = atomicAdd(a.head + 2, 1);
@@ -1113,8 +1167,11 @@ void launch_block_sq_inverse(const BlockArgs& a, double* tmp, hipStream_t stream
 bool launch_block_lds(const BlockArgs& a, int maxbs, int num_cu, hipStream_t stream)
 {
     if (maxbs > kLdsB) return false;
-    const int per_cu = (160 << 10) / (int)sizeof(BlkLds);
-    hipLaunchKernelGGL(block_lds_kernel, dim3(num_cu * per_cu), dim3(kWave), 0, stream, a);
+    auto launch = [&](auto kernel, size_t lds) {
+        hipLaunchKernelGGL(kernel, dim3(num_cu * (int)((160 << 10) / lds)), dim3(kWave), 0, stream, a);
+    };
+    launch(&block_lds_kernel<64, 24, 0>, sizeof(BlkLds<64, 24>));
+    launch(&block_lds_kernel<128, 36, 1>, sizeof(BlkLds<128, 36>));
     return true;
 }
 
