@@ -563,9 +563,14 @@ struct BlkLds {
     static constexpr int RT = ROWS / 16;   // rows per lane of the row-group layout
     static constexpr int kOwn = ROWS / kWave;  // rows per lane in row order
     static_assert(RT == 4 || RT == 8, "rows");
+    static constexpr int kWords = 2 * COLS * ROWS - kLdsRaw;
     union {
         double A[kLdsCols * kLdsRows];  // A(I,J), column-major: from the gather to the residual
-        int raw[kLdsRaw];               // index lists before sorting
+        struct {
+            int raw[kLdsRaw];  // index lists before their union
+            unsigned bits[kWords];
+        };
+        double sq[kLdsB * kLdsRows];  // squares of the residual
     };
     double r[kLdsB * kLdsRows];
     double x[kLdsB * kLdsCols];
@@ -575,6 +580,95 @@ struct BlkLds {
     int segs[kLdsCols], segoff[kLdsCols + 1];
     int sel[kLdsCols];
 };
+
+/* The sorted distinct values of the lists ind[ptr[l] .. ptr[l + 1]) of the
+ * nset indices l in `set` and of `extra` (when >= 0), less the sorted values
+ * excl[0..nexcl), into out: their number, or kBlkOverflow when the raw lists
+ * or the result (cap) have no room.  Through a bitmap over their range, or by
+ * a sort where that is wider than the bitmap: the sort's 15 to 28 stages took
+ * 7 to 8 us per set on the 256^2 grid of three fields. */
+template <class B>
+__device__ __forceinline__ int unique_union(B& w, const int* ptr, const int* ind, const int* set, int nset, int extra,
+                                            const int* excl, int nexcl, int* out, int cap)
+{
+    const int lane = W::lane();
+    const int nl = nset + (extra >= 0 ? 1 : 0);
+    int off = 0, lo = 0x7fffffff, hi = -1;
+    for (int base = 0; base < nl; base += kWave) {
+        const int t = base + lane;
+        int len = 0, e0 = 0;
+        if (t < nl) {
+            const int l = t < nset ? set[t] : extra;
+            e0 = ptr[l];
+            len = ptr[l + 1] - e0;
+        }
+        const int incl = W::scan_incl(len), total = W::bcast_last(incl);
+        if (off + total > kLdsRaw) return kBlkOverflow;
+        for (int e = 0; e < len; e += 8) {  // eight loads in flight
+            int v[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] = e + q < len ? ind[e0 + e + q] : 0;
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                if (e + q < len) {
+                    w.raw[off + incl - len + e + q] = v[q];
+                    lo = min(lo, v[q]);
+                    hi = max(hi, v[q]);
+                }
+        }
+        off += total;
+    }
+    __syncthreads();
+    if (off == 0) return 0;
+    lo = W::min_int(lo);
+    hi = W::max_int(hi);
+    int c = 0;
+    if (((hi - lo) >> 5) < B::kWords) {
+        const int words = ((hi - lo) >> 5) + 1;
+        for (int t = lane; t < words; t += kWave) w.bits[t] = 0u;
+        __syncthreads();
+        for (int e = lane; e < off; e += kWave) {
+            const int v = w.raw[e] - lo;
+            atomicOr(&w.bits[v >> 5], 1u << (v & 31));
+        }
+        __syncthreads();
+        for (int t = lane; t < nexcl; t += kWave) {
+            const int v = excl[t] - lo;
+            if (v >= 0 && v <= hi - lo) atomicAnd(&w.bits[v >> 5], ~(1u << (v & 31)));
+        }
+        __syncthreads();
+        for (int t0 = 0; t0 < words; t0 += kWave) {
+            unsigned b = t0 + lane < words ? w.bits[t0 + lane] : 0u;
+            const int cnt = __popc(b);
+            const int incl = W::scan_incl(cnt), chunk = W::bcast_last(incl);
+            if (c + chunk > cap) return kBlkOverflow;
+            int o = c + incl - cnt;
+            while (b) {
+                const int k = __ffs(b) - 1;
+                b &= b - 1u;
+                out[o++] = lo + ((t0 + lane) << 5) + k;
+            }
+            c += chunk;
+        }
+    } else {
+        const int nu = group_sort_unique<kWave>(w.raw, off, w.raw);
+        for (int base = 0; base < nu; base += kWave) {
+            const int t = base + lane;
+            const int u = t < nu ? w.raw[t] : 0;
+            bool keep = t < nu;
+            if (keep && nexcl > 0) {
+                const int q = lower_bound_i(excl, nexcl, u);
+                keep = !(q < nexcl && excl[q] == u);
+            }
+            const unsigned long long mask = W::ballot(keep);
+            if (c + __popcll(mask) > cap) return kBlkOverflow;
+            if (keep) out[c + __popcll(mask & W::lanes_below())] = u;
+            c += __popcll(mask);
+        }
+    }
+    __syncthreads();
+    return c;
+}
 
 /* Lane k of every row of 16 lanes, k a constant after unrolling. */
 template <int K = 0>
@@ -710,23 +804,8 @@ __device__ __forceinline__ int augment_lds(const BlockArgs& a, B& w, int col, in
     const int lane = W::lane();
     const int p = lower_bound_i(w.I, mi, col);
     const bool col_in = p < mi && w.I[p] == col;
-    const int nu = sorted_union(a.rp_ptr, a.rp_ind, w.I, mi, col_in ? -1 : col, w.raw, kLdsRaw, w.raw);
-    if (nu == kBlkOverflow) return kBlkOverflow;
-    int c = 0;
-    for (int base = 0; base < nu; base += kWave) {
-        const int t = base + lane;
-        const int u = t < nu ? w.raw[t] : 0;
-        bool keep = false;
-        if (t < nu) {
-            const int q = lower_bound_i(w.J, nj, u);
-            keep = !(q < nj && w.J[q] == u);
-        }
-        const unsigned long long mask = W::ballot(keep);
-        if (c + __popcll(mask) > kLdsU) return kBlkOverflow;
-        if (keep) w.cand[c + __popcll(mask & W::lanes_below())] = u;
-        c += __popcll(mask);
-    }
-    __syncthreads();
+    const int c = unique_union(w, a.rp_ptr, a.rp_ind, w.I, mi, col_in ? -1 : col, w.J, nj, w.cand, kLdsU);
+    if (c == kBlkOverflow) return kBlkOverflow;
     if (c == 0) return -1;
     /* one candidate per lane, two rounds at most; the scores stay in registers */
     double rho[2];
@@ -877,10 +956,8 @@ __device__ __forceinline__ bool block_column_lds(const BlockArgs& a, B& w, int c
     int st = 0, solves = 0, n = 0;
     double rn = 1.0e50;
     for (int step = -1; step < a.ns; ++step) {
-        const int mi = sorted_union(a.colptr, a.rowind, w.J, nj, -1, w.raw, kLdsRaw, w.raw);
-        if (mi == kBlkOverflow || mi > kLdsRows) return false;
-        for (int t = lane; t < mi; t += kWave) w.I[t] = w.raw[t];
-        __syncthreads();
+        const int mi = unique_union(w, a.colptr, a.rowind, w.J, nj, -1, nullptr, 0, w.I, kLdsRows);
+        if (mi == kBlkOverflow) return false;
         const int m = prefix_sizes(a.bsize, w.I, mi, w.fr);
         n = prefix_sizes(a.bsize, w.J, nj, w.fc);
         if (m > kLdsRows || n > kLdsCols) return false;
@@ -932,6 +1009,7 @@ __device__ __forceinline__ bool block_column_lds(const BlockArgs& a, B& w, int c
         for (int u = 0; u < kOwn; ++u)
 #pragma unroll
             for (int q = 0; q < kLdsB; ++q) r[u][q] = -((e0 >= 0 && lane + kWave * u == e0 + q) ? 1.0 : 0.0);
+#pragma unroll 4
         for (int jj = 0; jj < n; ++jj) {
 #pragma unroll
             for (int u = 0; u < kOwn; ++u) {
@@ -945,16 +1023,27 @@ __device__ __forceinline__ bool block_column_lds(const BlockArgs& a, B& w, int c
                     }
             }
         }
-        double sum = 0.0;
+        __syncthreads();  // A(I,J) is read
 #pragma unroll
         for (int q = 0; q < kLdsB; ++q)
             if (q < bk) {
 #pragma unroll
                 for (int u = 0; u < kOwn; ++u) {
-                    w.r[q * kLdsRows + lane + kWave * u] = r[u][q];
-                    const double sq = __dmul_rn(r[u][q], r[u][q]);
-                    for (int i = 0; i < min(m - kWave * u, kWave); ++i) sum = __dadd_rn(sum, W::lane_value(sq, i));
+                    const int i = lane + kWave * u;
+                    w.r[q * kLdsRows + i] = r[u][q];
+                    w.sq[q * kLdsRows + i] = i < m ? __dmul_rn(r[u][q], r[u][q]) : 0.0;
                 }
+            }
+        __syncthreads();
+        double sum = 0.0;  // formed by every lane; a row past |I| adds +0
+        for (int q = 0; q < bk; ++q)
+            for (int i = 0; i < m; i += 8) {
+                double2 d[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    d[k] = *reinterpret_cast<const double2*>(w.sq + q * kLdsRows + i + 2 * k);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) sum = __dadd_rn(__dadd_rn(sum, d[k].x), d[k].y);
             }
         __syncthreads();
         rn = sqrt(sum);
