@@ -1447,7 +1447,7 @@ __device__ __forceinline__ int ls_solve_rows64(const ScratchLayout& L, const Wav
  * stored entry of column j updates its row in order of j, as the dense
  * product does; the dense product's zero terms leave every nonzero residual
  * unchanged). */
-template <int G>
+template <int G, bool kHbm = true>
 __device__ __forceinline__ double residual_norm(const BuildArgs& a, const ScratchLayout& L, const WaveScratch& s,
                                                 int m, int n, bool dense,
                                                 const RowHash& h = RowHash{nullptr, 0, 0},
@@ -1533,9 +1533,9 @@ __device__ __forceinline__ double residual_norm(const BuildArgs& a, const Scratc
         }
     }
     double sum = 0.0;
-    if constexpr (G == kWave) {
+    if constexpr (G == kWave && kHbm) {
         /* the same sequential sum: each square formed on its row's lane,
-         * the terms taken in row order by readlane (no LDS round trip per
+         * the terms taken in row order by readlane (no memory round trip per
          * row on one lane) */
         for (int i0 = 0; i0 < m; i0 += kWave) {
             const int i = i0 + lane;
@@ -1545,13 +1545,18 @@ __device__ __forceinline__ double residual_norm(const BuildArgs& a, const Scratc
             for (int l = 0; l < cnt; ++l) sum = __dadd_rn(sum, Gr::lane_value(sq, l));
         }
     } else {
-        if (lane == 0) {
-            for (int i = 0; i < m; ++i) {
-                double v = s.r[i];
-                sum = __dadd_rn(sum, __dmul_rn(v, v));
+        /* formed by every lane, eight rows' reads in flight (a readlane per
+         * row, with its loop, took the random band's 64-lane bins 5% longer) */
+        for (int i0 = 0; i0 < m; i0 += 8) {
+            double v[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = s.r[min(i0 + k, m - 1)];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const double sq = i0 + k < m ? __dmul_rn(v[k], v[k]) : 0.0;  // + 0 past the last row
+                sum = __dadd_rn(sum, sq);
             }
         }
-        sum = Gr::bcast0(sum);
     }
     return sqrt(sum);
 }
@@ -2631,7 +2636,7 @@ __device__ __forceinline__ int solve_column(const BuildArgs& a, const ScratchLay
          * (dead after the LDS QR) */
         const double* Ad = (kTies && !dense) ? s.a0 : nullptr;
         const RowHash hR = (!kTies && !dense) ? row_hash_build<G>(s, L, m, a.A.nrows) : hI;
-        rn = residual_norm<G>(a, L, s, m, n, dense || Ad, hR, Ad);
+        rn = residual_norm<G, kTies>(a, L, s, m, n, dense || Ad, hR, Ad);
         if (kMixed && !(fabs(rn - a.epsilon) > kGuard * a.epsilon)) {
             redo = true;
             moved = step;
