@@ -16,9 +16,10 @@
  * Layout: the block matrix in HBM as block CSC (block e column-major at
  * val[voff[e]]), its block row pattern as CSR, (A_j^T A_j)^-1 per block
  * column, and the start pattern over block columns.  The working set of a
- * column (index sets, A(I,J) twice, the bk right-hand sides, residual) is a
- * per-wave slot in HBM sized for the largest column; the kernel is
- * persistent, the waves take block columns from an atomic counter.
+ * column (index sets, A(I,J), the bk right-hand sides, residual) is in LDS for
+ * small columns of small blocks, else (A(I,J) twice) a per-wave slot in HBM
+ * sized for the largest column; the kernels are persistent, the waves take
+ * block columns from an atomic counter.
  *
  * Order of operations: the 64-lane order for the QR (row r on lane r % 64,
  * fused partial sums, xor butterfly), dgemv's column order for the residual,
@@ -542,18 +543,22 @@ __device__ bool block_column(const BlockArgs& a, const BlockLayout& L, const Blk
     return true;
 }
 
-/* ---- block columns in LDS: |I| <= 64 and |J| <= 24 scalars, blocks to 4x4 ----
+/* ---- block columns in LDS: blocks to 4x4, |I| <= 64 and |J| <= 24 scalars
+ * (17 KB, 9 waves per CU), then |I| <= 128 and |J| <= 36 (44 KB) ----
  *
- * Almost every block column stays in these sizes (of the 65,536 on the 256^2
- * grid of three fields: FIG_SHARE).  With the working set in HBM each pass over
- * A(I,J), the residual or the scores waited for memory, the blocks of J were
- * gathered one column of A after another, and the register QR took four lane
- * moves per dot product.  Here the working set is 18 KB of LDS (9 waves per
- * CU), all blocks of J are gathered together, one per lane, the QR runs in the
- * row-group layout (in-lane sums, the right-hand sides one per row group), and
- * a candidate's numerator stays in registers.  FIG_BLOCK.  Bound by the latency
- * of those chains.  A column that outgrows it, or whose scores tie across the
- * cut, starts afresh in the HBM kernel: the same bits. */
+ * Of the 65,536 block columns on the 256^2 grid of three fields 65,490 stay in
+ * the first sizes.  With the working set in HBM each pass over A(I,J), the
+ * residual or the scores waited for memory, the blocks of J were gathered one
+ * column of A after another, and the register QR took four lane moves per dot
+ * product.  Here all blocks of J are gathered together, one per lane, the QR
+ * runs in the row-group layout (in-lane sums, the right-hand sides one per row
+ * group), and a candidate's numerator stays in registers.  On that grid the
+ * HBM kernel took 4.4 ms; the first LDS kernel takes 1.67 ms, the second 0.42
+ * ms (the latency of a few dozen columns) and the HBM kernel 0.05 ms for what
+ * is left.  Bound by VALU issue and the latency of those chains: 12 us of a
+ * solve's QR, 4 us of its memory round trips.  A column that outgrows the
+ * sizes, or whose scores tie across the cut, starts afresh in the next kernel:
+ * the same bits. */
 constexpr int kLdsB = 4, kLdsRaw = 512, kLdsU = 2 * kWave;
 
 /* Working set of |I| <= kLdsRows (64 or 128), |J| <= kLdsCols scalars. */
