@@ -27,6 +27,8 @@
  * of (A_j^T A_j)^-1 N, and the reference's own unfused sequential loops for
  * the trace term, the Frobenius sum, the mean and A_j^T A_j.
  */
+#include <type_traits>
+
 #include "device_common.h"
 #include "spai_host.h"
 
@@ -553,7 +555,7 @@ __device__ bool block_column(const BlockArgs& a, const BlockLayout& L, const Blk
  * product.  Here all blocks of J are gathered together, one per lane, the QR
  * runs in the row-group layout (in-lane sums, the right-hand sides one per row
  * group), and a candidate's numerator stays in registers.  On that grid the
- * HBM kernel took 4.4 ms; the first LDS kernel takes 1.67 ms, the second 0.42
+ * HBM kernel took 4.4 ms; the first LDS kernel takes 1.69 ms, the second 0.17
  * ms (the latency of a few dozen columns) and the HBM kernel 0.05 ms for what
  * is left.  Bound by VALU issue and the latency of those chains: 12 us of a
  * solve's QR, 4 us of its memory round trips.  A column that outgrows the
@@ -687,6 +689,15 @@ __device__ __forceinline__ double row_lane(double v, int k)
     }
 }
 
+/* f(I), f(I + 1), .. f(N - 1) with constant arguments, until one is false. */
+template <int I, int N, class F>
+__device__ __forceinline__ void steps(F f)
+{
+    if constexpr (I < N) {
+        if (f(std::integral_constant<int, I>{})) steps<I + 1, N>(f);
+    }
+}
+
 /* Approximative_Solution (block) in the row-group layout (lane 16 c + q: rows
  * q + 16 t of the columns c + 4 s); right-hand side c, the identity's column
  * at row e0 + c (none when e0 < 0), in slot NS of row group c.  Solution, or
@@ -719,9 +730,12 @@ __device__ __forceinline__ int block_solve_rows(B& w, int m, int n, int bk, int 
     for (int t = 0; t < RT; ++t) a[NS][t] = (c < bk && e0 >= 0 && q + 16 * t == e0 + c) ? 1.0 : 0.0;
     const int k = m < n ? m : n;
     bool zero_diag = false;
-#pragma unroll
-    for (int si = 0; si < NS; ++si) {
-        if (4 * si >= k) break;
+    /* step i = 4 si + ci, si a constant (by templates: the unrolled body is past
+     * the compiler's limit for eight rows per lane, and the array then lived in
+     * scratch memory: that launch took 0.42 instead of 0.17 ms) */
+    steps<0, NS>([&](auto slot) {
+        constexpr int si = decltype(slot)::value;
+        if (4 * si >= k) return false;
 #pragma unroll 1
         for (int ci = 0; ci < 4; ++ci) {
             const int i = 4 * si + ci;
@@ -765,7 +779,8 @@ __device__ __forceinline__ int block_solve_rows(B& w, int m, int n, int bk, int 
             }
             zero_diag |= rii == 0.0;
         }
-    }
+        return true;
+    });
     int st = 0;
     if (m < n) {
         st = COL_UNDERDET;
