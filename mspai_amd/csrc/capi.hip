@@ -1466,7 +1466,7 @@ static int run_static(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& wide
         for (int b = 0; b < kStaticKinds; ++b) {
             edges.capJ[b] = kStaticJ[b];
             edges.capI[b] = kStaticI[b];
-            edges.capSort[b] = 0x7fffffff;
+            edges.capSort[b] = kStaticJ[b] * kStaticI[b];  // |J| columns of at most |I| rows each
         }
         for (const Bin& b : wide) {
             edges.capJ[kStaticKinds] = b.L.capJ;

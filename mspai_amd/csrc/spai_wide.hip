@@ -137,11 +137,20 @@ __device__ __forceinline__ int block_scan(WideLds& w, int v, int* total)
 __device__ __forceinline__ unsigned row_slot(int row) { return ((unsigned)row * 0x9e3779b1u) >> 22; }
 static_assert(kHash == 1 << 10, "row_slot");
 
-/* Slot of `row`, added when new (-1: the table is full). */
+/* More distinct rows have arrived than the working set holds. */
+__device__ __forceinline__ bool rows_full(const WideLds& w)
+{
+    return __hip_atomic_load(&w.count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) > kI;
+}
+
+/* Slot of `row`, added when new.  -1: more rows than the working set holds,
+ * looked at every eighth probe (in a full table every insertion would
+ * otherwise walk all of it). */
 __device__ __forceinline__ int row_insert(WideLds& w, int row)
 {
     unsigned slot = row_slot(row);
     for (int probe = 0; probe < kHash; ++probe) {
+        if ((probe & 7) == 7 && rows_full(w)) break;
         const int old = atomicCAS(&w.key[slot], -1, row);
         if (old == -1) {
             const int k = atomicAdd(&w.count, 1);
@@ -202,7 +211,10 @@ __device__ __forceinline__ int index_set(const BuildArgs& a, WideLds& w, int n)
     }
     if (tid == 0) w.segoff[n] = total;
     __syncthreads();
-    for (int e = tid; e < total; e += kThreads) {
+    /* n columns with at most kI distinct rows each: a longer list cannot fit
+     * (inserting one of 10,000 entries took 1.9 ms) */
+    if (total > n * kI) return -1;
+    for (int e = tid; e < total && !rows_full(w); e += kThreads) {
         const int t = entry_column(w, n, e);
         row_insert(w, a.A.rowind[w.segs[t] + e - w.segoff[t]]);
     }
