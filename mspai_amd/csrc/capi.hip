@@ -1117,8 +1117,8 @@ static std::vector<Bin> bin_layouts(const mspai_ctx* ctx, int cap, int maxnew, b
         if ((needs & kNeedMixed) && table.mixed > 0 && (int)out.size() >= table.mixed) break;
         BinEdge e = table.e[t];
         if (e.group == kWideGroup) {
-            /* one column per workgroup in FP64 (also in a mixed build's
-             * chain); the QR update has one-wave kernels only */
+            /* one column per workgroup in FP64 (in a mixed build's chain with
+             * one refinement step); the QR update has one-wave kernels only */
             if (needs & kNeedQrUpdate) {
                 e.group = kWave;
             } else {
@@ -1367,6 +1367,7 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
             /* a bin the table runs in FP64 inside the mixed chain passes its
              * overflow on like the others and declines nothing */
             const int mode = bins[b].fp64 ? fp64_mode : 1;
+            a.refine = grp == kWideGroup;
             int per_cu = waves_per_cu(bins[b], mode);
             const ScratchLayout& L = bins[b].L;
             if ((rc = begin_launch(ctx, a, nullptr, mode, b, &bins[b]))) return rc;
@@ -1375,6 +1376,7 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
             HIPCHK(hipGetLastError());
             if (part == kFirstBin) return MSPAI_OK;
         }
+        a.refine = 0;
         a.status_or = COL_FALLBACK;
         a.save_state = 0;
         if (direct) {

@@ -1,0 +1,83 @@
+"""Precision 1 against an extended-precision solution of each column (64-bit
+mantissa): the refinement step must bring the values closer to it than the
+FP64 QR alone leaves them, whichever kernel finishes the column.
+
+A refined entry is off by its own rounding, at most u = 2^-53 of the column's
+largest entry, and by the rounding of the residual it was refined with (of
+the same size on these well-conditioned columns); an unrefined one by the
+rounding errors of |J| reflectors.  So the mean over many columns of the
+largest error of a column has to be below u, and below half of FP64's.
+"""
+import numpy as np
+import pytest
+import torch  # before the library: one HIP runtime per process  # noqa: F401
+
+from mspai_amd import gen
+
+pytestmark = pytest.mark.gpu
+U = 2.0 ** -53
+
+
+def extended_lstsq(A, b):
+    """Least-squares solution by Householder QR in long double."""
+    assert np.finfo(np.longdouble).nmant >= 63
+    A, b = A.astype(np.longdouble), b.astype(np.longdouble)
+    n = A.shape[1]
+    for i in range(n):
+        v = A[i:, i].copy()
+        v[0] += np.copysign(np.sqrt((v * v).sum()), v[0])
+        v /= np.sqrt((v * v).sum())
+        A[i:, i:] -= 2 * np.outer(v, v @ A[i:, i:])
+        b[i:] -= 2 * v * (v @ b[i:])
+    x = np.zeros(n, np.longdouble)
+    for i in range(n - 1, -1, -1):
+        x[i] = (b[i] - A[i, i + 1:] @ x[i + 1:]) / A[i, i]
+    return x
+
+
+def column_system(A, J, k):
+    sub = A[:, J]
+    I = np.unique(sub.indices)
+    return sub[I, :].toarray(), (I == k).astype(float), I.size
+
+
+def column_errors(A, M, cols):
+    """Largest error of each column's values, relative to its largest entry."""
+    out = []
+    for k in cols:
+        a, b = M.indptr[k], M.indptr[k + 1]
+        Ah, rhs, _ = column_system(A, M.indices[a:b], k)
+        x = extended_lstsq(Ah, rhs)
+        out.append(float(np.abs(M.data[a:b] - x).max() / np.abs(x).max()))
+    return np.array(out)
+
+
+def assert_refined(e0, e1):
+    print(f"   {e0.size} columns, mean error FP64 {e0.mean():.2e}, precision 1 {e1.mean():.2e}", flush=True)
+    assert e1.mean() <= U and e1.mean() <= 0.5 * e0.mean()
+
+
+def test_adaptive_columns_of_the_workgroup_kernel(gpu):
+    """Columns of more than 128 rows, which a mixed chain finishes in the
+    workgroup kernel."""
+    prob = gen.config3(n=32768, bw=2000)
+    opts = dict(epsilon=prob.epsilon, maxnew=prob.maxnew, max_impr_steps=prob.max_impr_steps)
+    b = gpu.Builder(0)
+    try:
+        b.upload(prob.A, prob.row_pattern())
+        b.set_pattern(prob.P)
+        M = []
+        for precision in (0, 1):
+            print(f"[refined workgroup columns precision={precision}]", flush=True)
+            b.set_bin_table(12, precision=precision)
+            b.build(binning=2, precision=precision, **opts)
+            M.append(b.download())
+        fallback = b.column_info()["status"] & 8
+    finally:
+        b.close()
+    assert np.array_equal(M[0].indptr, M[1].indptr) and np.array_equal(M[0].indices, M[1].indices)
+    rows = np.array([np.unique(prob.A[:, M[0].indices[M[0].indptr[k]:M[0].indptr[k + 1]]].indices).size
+                     for k in range(0, prob.n, 2)])
+    wide = [2 * t for t in np.flatnonzero(rows > 128) if not fallback[2 * t]][:80]
+    assert len(wide) >= 40
+    assert_refined(column_errors(prob.A, M[0], wide), column_errors(prob.A, M[1], wide))
