@@ -50,7 +50,8 @@ typedef struct {
     int use_mean;          /* -um  1: accept rho <= mean; 0: threshold = sum (1) */
     int qr;                /* -qr  0 = fresh QR per step, 2 = dense QR update (0) */
     int cache;             /* -cs  device pattern->R cache entries, 0 = off (0) */
-    int precision;         /* GPU: 0 = FP64, 1 = FP32 QR + FP64 refinement (0) */
+    int precision;         /* GPU: 0 = FP64, 1 = FP32 QR + FP64 refinement (0); in static builds, the
+                              adjoint and the widest size bin an FP64 QR + one step of refinement */
     int binning;           /* GPU: 1 = default size bins, 2 = autotuned bins (mspai_autotune),
                               0 = one generic bin (1) */
     int verbose;           /* -vb */

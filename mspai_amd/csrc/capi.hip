@@ -1422,13 +1422,19 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
 }
 
 /* The bins of static builds and the adjoint: the kinds of the given-pattern
- * kernels, then one 64-lane LDS bin of |J| <= 40, |I| <= 128 for the wider
- * columns (`wide`: its layout, none when the kinds hold every column), then
- * the generic kernel. */
-static std::vector<Bin> static_wide_bin(const mspai_ctx* ctx, int cap, const ScratchLayout& G, int needs)
+ * kernels, then bins for the wider columns (returned here), then the generic
+ * kernel.  A 64-lane LDS bin takes |J| <= 40, |I| <= 128, the workgroup kernel
+ * |I| <= 384 (builds only).  A build at precision 1 has the workgroup kernel
+ * alone, which refines its solutions as the kinds do, at the price of the
+ * 64-lane bin's: 6,000 columns of |J| 20 to 40, |I| 60 to 130 take 1.54 ms
+ * there, 1.56 ms unrefined in both bins (6,000 of |I| 110 to 240: 1.83 and 2.23
+ * ms, 3.76 ms with the generic kernel after the 64-lane bin). */
+static std::vector<Bin> static_wide_bins(const mspai_ctx* ctx, int cap, const ScratchLayout& G, int needs, bool refine)
 {
-    static const BinTable kWide = {"g64", 1, {{64, 40, 128, 512, 1024, 0}}};
-    return bin_layouts(ctx, cap, 1, false, G, kWide, needs);
+    static const BinTable kWide = {"g64-g64x384", 2, {{64, 40, 128, 512, 1024, 0}, {512, 40, 384, 4096, 8192, 0}}};
+    static const BinTable kRefined = {"g64x384", 1, {{512, 40, 384, 4096, 8192, 0}}};
+    static const BinTable kBack = {"g64", 1, {{64, 40, 128, 512, 1024, 0}}};
+    return bin_layouts(ctx, cap, 1, false, G, needs & kNeedBackward ? kBack : refine ? kRefined : kWide, needs);
 }
 
 /* Launch a static build (mode 0) or the adjoint (mode 2) over the columns
@@ -1438,7 +1444,7 @@ static std::vector<Bin> static_wide_bin(const mspai_ctx* ctx, int cap, const Scr
  * index and the routing kernel is not run (71 to 120 us of 0.26 million
  * columns); lists of more uneven columns are routed, so that short ones run
  * eight to a wave.  *first: that kind, or -1.  Queues and counters as in
- * run_chain, queue b < kStaticKinds for the kinds, then the wide bin's, then
+ * run_chain, queue b < kStaticKinds for the kinds, then the wide bins', then
  * the generic kernel's. */
 static int run_static(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& wide, const ScratchLayout& G, int gwaves,
                       int mode, bool refine, int n, int longest, double mean, int* first)
@@ -1470,10 +1476,10 @@ static int run_static(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& wide
             edges.capI[b] = kStaticI[b];
             edges.capSort[b] = kStaticJ[b] * kStaticI[b];  // |J| columns of at most |I| rows each
         }
-        for (const Bin& b : wide) {
-            edges.capJ[kStaticKinds] = b.L.capJ;
-            edges.capI[kStaticKinds] = b.L.capI;
-            edges.capSort[kStaticKinds] = b.L.capSid;
+        for (int b = 0; b < (int)wide.size(); ++b) {
+            edges.capJ[kStaticKinds + b] = wide[b].L.capJ;
+            edges.capI[kStaticKinds + b] = wide[b].L.capI;
+            edges.capSort[kStaticKinds + b] = wide[b].L.capSid;
         }
         ctx->was_routed = true;
         a.stamp = ctx->d_ts + kStampRoute;
@@ -1505,11 +1511,13 @@ static int run_static(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& wide
         const int t = kStaticKinds + b;
         a.overflow = q + (size_t)(t + 1) * n;
         a.n_overflow = counts + t + 1;
+        a.refine = refine && wide[b].group == kWideGroup;
         if ((rc = begin_launch(ctx, a, nullptr, mode, t, &wide[b]))) return rc;
         launch_binned(a, wide[b].L, wide[b].group, mode, q + (size_t)t * n, counts + t, heads + t,
                       ctx->num_cu * waves_per_cu(wide[b], mode), ctx->stream, wide[b].wcap);
         HIPCHK(hipGetLastError());
     }
+    a.refine = 0;
     a.overflow = q;  // never written: the generic layout holds every column
     a.n_overflow = counts + 7;
     if ((rc = begin_launch(ctx, a, "generic (HBM working set)", mode, -1, nullptr))) return rc;
@@ -1645,7 +1653,7 @@ extern "C" int mspai_build(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* 
      * which only the adaptive builds' kernels keep) */
     const bool given = given_pattern_build(ctx, opts);
     if (given) {
-        bins = static_wide_bin(ctx, cap, G, needs & ~kNeedMixed);
+        bins = static_wide_bins(ctx, cap, G, needs & ~kNeedMixed, opts->precision == 1);
         ctx->last_table = table_for(ctx, opts);
     } else if (opts->binning && !ctx->d_up_ptr) {  // an upper pattern runs unbinned
         int t = table_for(ctx, opts);
@@ -1820,7 +1828,7 @@ extern "C" int mspai_build_noalloc(mspai_ctx* ctx, const mspai_opts* opts, int* 
     const ScratchLayout G = generic_layout(ctx, cap, opts->maxnew, adaptive, needs);
     std::vector<Bin> bins, fbins;
     if (given_pattern_build(ctx, opts)) {
-        fbins = static_wide_bin(ctx, cap, G, needs & ~kNeedMixed);
+        fbins = static_wide_bins(ctx, cap, G, needs & ~kNeedMixed, opts->precision == 1);
     } else if (opts->binning && !ctx->d_up_ptr) {  // an upper pattern runs unbinned
         int t = table_for(ctx, opts);
         bins = bin_layouts(ctx, cap, opts->maxnew, adaptive, G, kTables[t], needs);
@@ -1949,7 +1957,7 @@ extern "C" int mspai_backward(mspai_ctx* ctx, const mspai_opts* opts, const doub
     const int n = ctx->ncols;
     const int cap = ctx->cap;
     const ScratchLayout G = generic_layout(ctx, cap, 1, false, kNeedBackward);
-    const std::vector<Bin> wide = opts->binning ? static_wide_bin(ctx, cap, G, kNeedBackward) : std::vector<Bin>{};
+    const std::vector<Bin> wide = opts->binning ? static_wide_bins(ctx, cap, G, kNeedBackward, false) : std::vector<Bin>{};
     int gwaves = 0;
     if ((rc = prepare_generic(ctx, G, &gwaves))) return rc;
     if ((rc = start_build(ctx))) return rc;

@@ -10,6 +10,7 @@ largest error of a column has to be below u, and below half of FP64's.
 """
 import numpy as np
 import pytest
+import scipy.sparse as sp
 import torch  # before the library: one HIP runtime per process  # noqa: F401
 
 from mspai_amd import gen
@@ -81,3 +82,52 @@ def test_adaptive_columns_of_the_workgroup_kernel(gpu):
     wide = [2 * t for t in np.flatnonzero(rows > 128) if not fallback[2 * t]][:80]
     assert len(wide) >= 40
     assert_refined(column_errors(prob.A, M[0], wide), column_errors(prob.A, M[1], wide))
+
+
+def given_pattern_problem(lens, nnz, band, seed=0, n=400):
+    """n columns of `nnz` entries within `band` of a dominant diagonal; column
+    k's pattern holds lens[k % len(lens)] indices around k."""
+    rng = np.random.Generator(np.random.PCG64(seed))
+    rows, cols, vals, ptr, ind = [], [], [], [0], []
+    for j in range(n):
+        near = np.arange(max(0, j - band), min(n, j + band + 1))
+        r = np.union1d(rng.choice(near, size=min(near.size, nnz), replace=False), [j])
+        v = rng.standard_normal(r.size)
+        v[r == j] = 4.0
+        rows.append(r), cols.append(np.full(r.size, j)), vals.append(v)
+        want = lens[j % len(lens)]
+        near = np.setdiff1d(np.arange(max(0, j - want), min(n, j + want + 1)), [j])
+        ind.append(np.union1d(rng.choice(near, size=want - 1, replace=False), [j]).astype(np.int64))
+        ptr.append(ptr[-1] + want)
+    A = gen._csc(np.concatenate(rows), np.concatenate(cols), np.concatenate(vals), (n, n))
+    P = sp.csc_matrix((np.ones(ptr[-1]), np.concatenate(ind), ptr), shape=(n, n))
+    return gen.Problem("given", A, P, None, max_impr_steps=0)
+
+
+STATIC = {  # pattern lengths, entries of a column; the columns' |I|
+    "kinds": ((7, 15, 31), 2, (1, 64)),
+    "rows_65_to_128": ((20, 24, 30), 5, (65, 128)),
+    "columns_32_to_40": ((32, 36, 40), 2, (33, 128)),
+    "rows_129_to_384": ((24, 36, 40), 14, (129, 384)),
+}
+
+
+@pytest.mark.parametrize("name", sorted(STATIC))
+def test_static_columns(gpu, name):
+    lens, nnz, (lo, hi) = STATIC[name]
+    prob = given_pattern_problem(lens, nnz, 100)
+    b = gpu.Builder(0)
+    try:
+        b.upload(prob.A, prob.row_pattern())
+        b.set_pattern(prob.P)
+        M = []
+        for precision in (0, 1):
+            print(f"[refined static {name} precision={precision}]", flush=True)
+            b.build(max_impr_steps=0, precision=precision)
+            M.append(b.download())
+    finally:
+        b.close()
+    size = [column_system(prob.A, M[0].indices[M[0].indptr[k]:M[0].indptr[k + 1]], k)[2] for k in range(prob.n)]
+    cols = [k for k in range(prob.n) if lo <= size[k] <= hi][::3]
+    assert len(cols) >= 60
+    assert_refined(column_errors(prob.A, M[0], cols), column_errors(prob.A, M[1], cols))
