@@ -179,9 +179,9 @@ int mspai_result_values_device(mspai_ctx* ctx, double* d_out);
  * d_gC = dL/dC (device, nnz(C) doubles in C's CSC order) and, when a target
  * is set and d_gB is not NULL, d_gB = dL/dB (nnz(B) doubles).  Per column:
  * r = b - C(I,J) m, R^T R lambda = g, dL/dC(i,j) = r_i lambda_j -
- * (C lambda)_i m_j, dL/db = C lambda, with the QR recomputed (FP64, or FP32
- * with refinement when opts->precision is 1).  No counterpart in the
- * reference (it has no derivatives); MSPAI probing weights rho enter through
+ * (C lambda)_i m_j, dL/db = C lambda, with the QR recomputed in FP64 (when
+ * opts->precision is 1 lambda takes one refinement step in columns of |J| <=
+ * 40, |I| <= 128).  No counterpart in the reference (it has no derivatives); MSPAI probing weights rho enter through
  * C's and B's probe rows, so dL/drho follows from gC and gB by the chain rule.
  * Accumulation into gC uses atomics, so its last bits depend on timing.
  */

@@ -1511,7 +1511,7 @@ static int run_static(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& wide
         const int t = kStaticKinds + b;
         a.overflow = q + (size_t)(t + 1) * n;
         a.n_overflow = counts + t + 1;
-        a.refine = refine && wide[b].group == kWideGroup;
+        a.refine = refine && (back || wide[b].group == kWideGroup);
         if ((rc = begin_launch(ctx, a, nullptr, mode, t, &wide[b]))) return rc;
         launch_binned(a, wide[b].L, wide[b].group, mode, q + (size_t)t * n, counts + t, heads + t,
                       ctx->num_cu * waves_per_cu(wide[b], mode), ctx->stream, wide[b].wcap);

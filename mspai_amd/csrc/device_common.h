@@ -101,7 +101,7 @@ struct BuildArgs {
     double epsilon;
     int maxnew, ns, use_mean;
     int cap;                // capacity of one output column
-    int refine;             // workgroup kernel: one refinement step on a finished column's solution (precision 1)
+    int refine;             // precision 1: one refinement step in the workgroup kernel and in the adjoint's 64-lane bin
     int direct;             // static build: column k's outputs at p_ptr[k] (M has the start pattern) instead of k*cap
     int nqueue;             // columns 0..nqueue of a launch without a queue
     unsigned long long* stamp;  // start time of this launch

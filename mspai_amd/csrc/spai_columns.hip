@@ -2055,7 +2055,10 @@ __device__ __forceinline__ void count_solve(const BuildArgs& a, const WaveScratc
 }
 
 /* The adjoint of one column of M (pattern in p_ptr/p_ind, values m_in) for
- * columns wider than the given-pattern kernels take: |J| up to the layout's. */
+ * columns wider than the given-pattern kernels take: |J| up to the layout's.
+ * With a.refine (precision 1, the 64-lane bin) lambda takes the refinement
+ * step that those kernels take: lambda += (R^T R)^-1 (g - C^T C lambda), when
+ * it is at most 1e-10 max|lambda|. */
 template <int G, bool kHbm>
 __device__ __forceinline__ int backward_column(const BuildArgs& a, const ScratchLayout& L, const WaveScratch& s,
                                                int col)
@@ -2080,9 +2083,29 @@ __device__ __forceinline__ int backward_column(const BuildArgs& a, const Scratch
     if (ls_solve<G>(L, s, m, n) & (COL_SINGULAR | COL_UNDERDET)) return kDone;
     /* r = b - C m (into s.r) */
     csc_apply<G>(a, L, s, m, n, s.y, s.b0, s.r, false);
+    if (!kHbm && a.refine) {
+        for (int i = lane; i < n; i += G) s.z[i] = s.g[i];
+        __syncthreads();
+    }
     normal_solve<G>(s.aqr, ld, s.g, n);
     /* s = C lambda (into s.b0) */
     csc_apply<G>(a, L, s, m, n, s.g, nullptr, s.b0, false);
+    if (!kHbm && a.refine) {
+        csc_apply_t<G>(a, L, s, m, n, s.b0, s.b, false);
+        for (int i = lane; i < n; i += G) s.b[i] = s.z[i] - s.b[i];
+        __syncthreads();
+        normal_solve<G>(s.aqr, ld, s.b, n);
+        double lmx = 0.0;
+        for (int i = lane; i < n; i += G) lmx = fmax(lmx, fabs(s.g[i]));
+        lmx = Gr::max(lmx);
+        bool large = false;
+        for (int i = lane; i < n; i += G) large |= !(fabs(s.b[i]) <= 1e-10 * lmx);
+        if (Gr::ballot(large) == 0ull) {
+            for (int i = lane; i < n; i += G) s.g[i] += s.b[i];
+            __syncthreads();
+            csc_apply<G>(a, L, s, m, n, s.g, nullptr, s.b0, false);
+        }
+    }
     /* dL/dC_ij += r_i lambda_j - s_i m_j over the stored entries of J (the
      * column segments build_I left) */
     const int total = s.segoff[n];

@@ -131,3 +131,64 @@ def test_static_columns(gpu, name):
     cols = [k for k in range(prob.n) if lo <= size[k] <= hi][::3]
     assert len(cols) >= 60
     assert_refined(column_errors(prob.A, M[0], cols), column_errors(prob.A, M[1], cols))
+
+
+def extended_adjoint(A, g):
+    """A lambda with A^T A lambda = g, by the R of a long double QR."""
+    A0, A = A.astype(np.longdouble), A.astype(np.longdouble)
+    n = A.shape[1]
+    for i in range(n):
+        v = A[i:, i].copy()
+        v[0] += np.copysign(np.sqrt((v * v).sum()), v[0])
+        v /= np.sqrt((v * v).sum())
+        A[i:, i:] -= 2 * np.outer(v, v @ A[i:, i:])
+    lam = g.astype(np.longdouble)
+    for i in range(n):
+        lam[i] = (lam[i] - A[:i, i] @ lam[:i]) / A[i, i]
+    for i in range(n - 1, -1, -1):
+        lam[i] = (lam[i] - A[i, i + 1:n] @ lam[i + 1:]) / A[i, i]
+    return A0 @ lam
+
+
+@pytest.mark.parametrize("name", ["kinds", "rows_65_to_128", "columns_32_to_40"])
+def test_adjoint_columns(gpu, name):
+    """dL/dB(:, k) = C lambda over I, one column's own values: a target with
+    every row of I in it gives all of them.  The step removes what the QR and
+    the two triangular solves left; what remains is the rounding of C lambda
+    and C^T (C lambda): on average below three quarters of FP64's error."""
+    lens, nnz, (lo, hi) = STATIC[name]
+    prob = given_pattern_problem(lens, nnz, 100, n=300)
+    n, P = prob.n, prob.P
+    J = [P.indices[P.indptr[k]:P.indptr[k + 1]] for k in range(n)]
+    I = [np.unique(prob.A[:, J[k]].indices) for k in range(n)]
+    B = gen._csc(np.concatenate(I), np.repeat(np.arange(n), [i.size for i in I]),
+                 np.concatenate([(i == k) + 0.0 for k, i in enumerate(I)]), (n, n))
+    assert B.nnz == sum(i.size for i in I)  # the zeros are stored
+    g = np.random.Generator(np.random.PCG64(5)).standard_normal(P.nnz)
+    b = gpu.Builder(0)
+    gbs = []
+    try:
+        b.upload(prob.A, prob.row_pattern())
+        b.set_pattern(P)
+        b.set_target(B)
+        gm = torch.tensor(g, device="cuda")
+        gc = torch.empty(prob.A.nnz, dtype=torch.float64, device="cuda")
+        gb = torch.empty(B.nnz, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        for precision in (0, 1):
+            print(f"[refined adjoint {name} precision={precision}]", flush=True)
+            b.build(max_impr_steps=0, precision=precision)
+            b.backward_device(gm.data_ptr(), gc.data_ptr(), gb.data_ptr(), precision=precision)
+            gbs.append(gb.cpu().numpy())
+    finally:
+        b.close()
+    e = [[], []]
+    for k in [k for k in range(n) if lo <= I[k].size <= hi][::3]:
+        exact = extended_adjoint(prob.A[:, J[k]][I[k], :].toarray(), g[P.indptr[k]:P.indptr[k + 1]])
+        for p in (0, 1):
+            d = gbs[p][B.indptr[k]:B.indptr[k + 1]] - exact
+            e[p].append(float(np.abs(d).max() / np.abs(exact).max()))
+    assert len(e[0]) >= 50
+    e0, e1 = np.mean(e[0]), np.mean(e[1])
+    print(f"   {len(e[0])} columns, mean error FP64 {e0:.2e}, precision 1 {e1:.2e}", flush=True)
+    assert e1 <= 0.75 * e0
