@@ -192,8 +192,12 @@ int mspai_backward(mspai_ctx* ctx, const mspai_opts* opts, const double* d_gM, d
  * Autotuner of the size bins (no counterpart in the reference): builds the
  * uploaded problem with each candidate bin table (lane-group widths, |J| and
  * |I| edges, resident-wave caps), `repeats` timed runs each after one warm-up,
- * and keeps the fastest for later builds with opts->binning == 2.  Results do
- * not depend on the table.  A new mspai_upload_csc clears the choice.
+ * and keeps the fastest for later builds with opts->binning == 2.  The pattern
+ * of M does not depend on the table, nor do its values in FP64.  Static builds
+ * (max_impr_steps 0) and the adjoint run on kernels of their own whatever the
+ * table, unless the build keeps work counters or the cache or has an upper
+ * pattern: on such options the build is timed once and the choice kept.  A new
+ * mspai_upload_csc clears the choice.
  */
 #define MSPAI_MAX_TUNE 32
 typedef struct {
@@ -205,7 +209,7 @@ typedef struct {
 int mspai_autotune(mspai_ctx* ctx, const mspai_opts* opts, int repeats, mspai_tune_report* report);
 
 /* Sets the bin table that builds of `precision` (0 FP64, 1 mixed) with
- * opts->binning == 2 use, as the autotuner would (no counterpart in the
+ * opts->binning == 2 use (adaptive ones: see mspai_autotune), as the autotuner would (no counterpart in the
  * reference: for tests and for callers that tune once and store the choice).
  * `name` (32 bytes, may be NULL) receives the table's name, `ntables` (may be
  * NULL) the number of tables; table < 0 only reports that number.  Mixed

@@ -2002,7 +2002,9 @@ extern "C" int mspai_autotune(mspai_ctx* ctx, const mspai_opts* opts, int repeat
     double best_ms = 1e300;
     if (report) std::memset(report, 0, sizeof(*report));
     const int prec = o.precision == 1 ? 1 : 0;
-    for (int t = 0; t < kNumTables && t < MSPAI_MAX_TUNE; ++t) {
+    const int kept = ctx->tuned_table[prec];
+    bool given = false;
+    for (int t = 0; t < kNumTables && !given && t < MSPAI_MAX_TUNE; ++t) {
         if ((prec == 1 && kTables[t].count == 0) || (prec == 0 && (kTables[t].mixed > 0 || kTables[t].fp64mask))) {
             /* the mixed kernels run in size bins: a bin-less table is all
              * FP64; a limit on the mixed chain changes nothing in FP64 */
@@ -2020,13 +2022,21 @@ extern "C" int mspai_autotune(mspai_ctx* ctx, const mspai_opts* opts, int repeat
             }
             if (r > 0) tmin = std::min(tmin, st.solve_ms);
         }
+        /* the given-pattern kernels do not depend on the table: timed once,
+         * and what adaptive builds use stays as it was */
+        given = given_pattern_build(ctx, &o);
+        if (given) {
+            ctx->tuned_table[prec] = kept;
+            t = best = table_for(ctx, &o);
+            for (int u = 0; report && u < std::min(kNumTables, MSPAI_MAX_TUNE); ++u) report->candidate_ms[u] = -1.0;
+        }
         if (report) report->candidate_ms[t] = tmin;
         if (tmin < best_ms) {
             best_ms = tmin;
             best = t;
         }
     }
-    ctx->tuned_table[prec] = best;
+    if (!given) ctx->tuned_table[prec] = best;
     if (report) {
         report->ncandidates = std::min(kNumTables, MSPAI_MAX_TUNE);
         report->chosen = best;
