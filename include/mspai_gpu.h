@@ -195,9 +195,9 @@ int mspai_backward(mspai_ctx* ctx, const mspai_opts* opts, const double* d_gM, d
  * and keeps the fastest for later builds with opts->binning == 2.  The pattern
  * of M does not depend on the table, nor do its values in FP64.  Static builds
  * (max_impr_steps 0) and the adjoint run on kernels of their own whatever the
- * table, unless the build keeps work counters or the cache or has an upper
- * pattern: on such options the build is timed once and the choice kept.  A new
- * mspai_upload_csc clears the choice.
+ * table, unless the build keeps the cache or has an upper pattern: on such
+ * options the build is timed once and the choice kept.  A new mspai_upload_csc
+ * clears the choice.
  */
 #define MSPAI_MAX_TUNE 32
 typedef struct {

@@ -1455,7 +1455,8 @@ static int run_static(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& wide
     int* heads = ctx->d_counter + 8;
     int* q = ctx->d_queues;
     int rc;
-    ctx->lwork_valid = false;
+    ctx->lwork_valid = a.work != nullptr;
+    if (a.work) HIPCHK(hipMemsetAsync(ctx->d_lwork, 0, kMaxLaunch * kLaunchStat * sizeof(double), ctx->stream));
     a.status_or = 0;
     a.save_state = 0;
     const size_t tie_need = tie_bytes_needed(ctx, wide, wide, false, mode);
@@ -1602,10 +1603,10 @@ static int prepare_generic(mspai_ctx* ctx, const ScratchLayout& G, int* gwaves)
     return ensure_scratch(ctx, (size_t)w * G.per_wave);
 }
 
-/* A static build with size bins that keeps neither counters nor the cache. */
+/* A static build with size bins that does not keep the cache. */
 static bool given_pattern_build(const mspai_ctx* ctx, const mspai_opts* o)
 {
-    return o->max_impr_steps == 0 && o->binning && !o->counters && !(o->cache > 0 && o->precision == 0) &&
+    return o->max_impr_steps == 0 && o->binning && !(o->cache > 0 && o->precision == 0) &&
            !ctx->d_up_ptr && ctx->p_base0;
 }
 
@@ -1649,8 +1650,8 @@ extern "C" int mspai_build(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* 
     const ScratchLayout G = generic_layout(ctx, cap, opts->maxnew, adaptive, needs);
     std::vector<Bin> bins, fbins;
     /* static builds take the given-pattern kernels, FP64 under either
-     * precision, whatever the bin table (not with counters or the cache,
-     * which only the adaptive builds' kernels keep) */
+     * precision, whatever the bin table (not with the cache, which only the
+     * adaptive builds' kernels keep) */
     const bool given = given_pattern_build(ctx, opts);
     if (given) {
         bins = static_wide_bins(ctx, cap, G, needs & ~kNeedMixed, opts->precision == 1);
