@@ -26,6 +26,7 @@
 using namespace mspai;
 
 constexpr int kMaxBins = 5;
+constexpr int kQueues = 9;  // work queues of ncols entries: those of the FP64 chain first, of the mixed chain last (run_chain)
 constexpr int kMaxLaunch = 2 * kMaxBins + 2;  // column-kernel launches of one build: mixed bins, FP64 bins, generic
 /* Time stamps of a build, written by the kernels themselves as they start (an
  * event between two launches holds the stream for several microseconds): one
@@ -249,7 +250,7 @@ struct mspai_ctx {
     long long pattern_nnz = -1;  // nnz of the last built M's pattern (kept across value updates)
     size_t Mcap = 0;
     // queues and scratch
-    int* d_queues = nullptr;   // (kMaxBins + 1) queues of ncols entries
+    int* d_queues = nullptr;   // kQueues queues of ncols entries
     int* d_counter = nullptr;  // FP64 queues: [0..8) lengths, [8..16) heads; [16..24) routed lengths;
                                // mixed queues: [24..32) lengths, [32..40) heads
     int* h_counter = nullptr;  // pinned host copy of d_counter, [63] = nnz(M) of the last build
@@ -837,7 +838,7 @@ static int ensure_outputs(mspai_ctx* ctx, int cap)
     HIPCHK(hipMalloc((void**)&ctx->d_Mptr, (n + 1) * sizeof(int)));
     HIPCHK(hipMalloc((void**)&ctx->d_Mind, n * cap * sizeof(int)));
     HIPCHK(hipMalloc((void**)&ctx->d_Mval, n * cap * sizeof(double)));
-    HIPCHK(hipMalloc((void**)&ctx->d_queues, (2 * kMaxBins + 1) * n * sizeof(int)));
+    HIPCHK(hipMalloc((void**)&ctx->d_queues, kQueues * n * sizeof(int)));
     ctx->cap = cap;
     ctx->out_cols = n;
     ctx->Mcap = n * cap;
@@ -1291,8 +1292,10 @@ enum ChainPart { kWholeChain, kFirstBin, kRestOfChain };
 /* Launch routing and the bin chain over the columns whose patterns are in
  * a.p_ptr/p_ind.  `bins` are the mixed chain's bins in a mixed build (else
  * the FP64 chain's), `fbins` the FP64 chain's.  Queues: FP64 queue b at
- * d_queues + b*n (b = 0..nf, nf = generic), mixed queue b at d_queues +
- * (kMaxBins + 1 + b)*n.  Routing fills the first queues; a bin's overflow
+ * d_queues + b*n (b = 0..nf, nf = generic), mixed queue b of nb at d_queues +
+ * (kQueues - nb + b)*n.  The two overlap in FP64 queues 4 and 5 (nb = 5) or 5
+ * (nb = 4): no mixed launch but the last writes an FP64 queue other than 0,
+ * and that one reads the last mixed queue alone.  Routing fills the first queues; a bin's overflow
  * appends to the next queue of its chain; the mixed chain ends in FP64
  * queue 0, which also takes the columns the mixed guards decline.  Columns
  * go on from the step they reached (save_state) except in the adjoint and
@@ -1320,7 +1323,7 @@ static int run_chain(mspai_ctx* ctx, BuildArgs& a, const std::vector<Bin>& bins,
     int* mcounts = ctx->d_counter + 24;
     int* mheads = ctx->d_counter + 32;
     int* fq = ctx->d_queues;
-    int* mq = ctx->d_queues + (size_t)(kMaxBins + 1) * n;
+    int* mq = ctx->d_queues + (size_t)(kQueues - nb) * n;  // (mixed builds)
     int rc;
     ctx->lwork_valid = a.work != nullptr;
     if (a.work) HIPCHK(hipMemsetAsync(ctx->d_lwork, 0, kMaxLaunch * kLaunchStat * sizeof(double), ctx->stream));
@@ -1753,7 +1756,7 @@ extern "C" int mspai_build(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* 
             return rc;
         /* the tiles' sums go to a queue that is empty: the first one, or with
          * the chain not ended the mixed one that the straight chain leaves */
-        int* const sums = ctx->d_queues + (alone && mixed ? (size_t)(kMaxBins + 1) * n : 0);
+        int* const sums = ctx->d_queues + (alone && mixed ? (size_t)(kQueues - (int)bins.size()) * n : 0);
         if ((rc = finish(sums))) return rc;
         const int* hc = ctx->h_counter;
         int moved = 0;
@@ -1811,15 +1814,15 @@ extern "C" int mspai_build_noalloc(mspai_ctx* ctx, const mspai_opts* opts, int* 
         return fail(ctx, MSPAI_ERR_CAPACITY, "build_noalloc: max_nnz must be at least ncols * (max |J0| + mn * ns) = " +
                                                  std::to_string(n * cap));
     /* carve the static array: the build's fixed buffers first, then the
-     * tie buffers of the size bins, the scan workspace, and what is left
-     * for the generic kernel's working sets */
+     * tie buffers of the size bins, and what is left for the generic kernel's
+     * working sets */
     size_t off = 0;
     auto take = [&](size_t bytes) {
         size_t at = off;
         off = align_up(off + bytes, 256);
         return ctx->d_noalloc + at;
     };
-    const size_t fixed = align_up(64 * sizeof(int), 256) + align_up((2 * kMaxBins + 1) * n * sizeof(int), 256) +
+    const size_t fixed = align_up(64 * sizeof(int), 256) + align_up(kQueues * n * sizeof(int), 256) +
                          align_up(n * sizeof(int), 256) + align_up(n * cap * sizeof(int), 256) +
                          align_up(n * cap * sizeof(double), 256) + align_up(n * sizeof(double), 256) +
                          2 * align_up(n * sizeof(int), 256);
@@ -1839,10 +1842,7 @@ extern "C" int mspai_build_noalloc(mspai_ctx* ctx, const mspai_opts* opts, int* 
     }
     const bool mixed = opts->precision == 1 && !bins.empty() && !qrup;
     const size_t tie = align_up(tie_bytes_needed(ctx, bins, fbins, mixed, qrup ? 4 : 0), 256);
-    size_t cub = 0;
-    hipcub::DeviceScan::InclusiveSum(nullptr, cub, (const int*)nullptr, (int*)nullptr, (int)n, ctx->stream);
-    cub = align_up(std::max<size_t>(cub, 256), 256);
-    if (fixed + tie + cub + G.per_wave > kNoAllocBytes)
+    if (fixed + tie + G.per_wave > kNoAllocBytes)
         return fail(ctx, MSPAI_ERR_CAPACITY, "build_noalloc: the problem needs more than the " +
                                                  std::to_string(MSPAI_NOALLOC_SCRATCH_MIB) + " MiB scratch array");
     /* the context's own buffers step aside for the call */
@@ -1850,14 +1850,13 @@ extern "C" int mspai_build_noalloc(mspai_ctx* ctx, const mspai_opts* opts, int* 
         int *counter, *queues, *m_len, *m_idx, *nsolve, *status, *Mptr, *Mind;
         double *m_val, *res, *work, *Mval;
         char *tie, *scr;
-        void* cub;
-        size_t tie_bytes, cub_bytes, scr_bytes, Mcap, out_cols;
+        size_t tie_bytes, scr_bytes, Mcap, out_cols;
         int cap;
     } sv{ctx->d_counter, ctx->d_queues, ctx->d_m_len, ctx->d_m_idx, ctx->d_nsolve, ctx->d_status, ctx->d_Mptr,
-         ctx->d_Mind, ctx->d_m_val, ctx->d_res, ctx->d_work, ctx->d_Mval, ctx->d_tie, ctx->d_scratch, ctx->d_cub,
-         ctx->tie_bytes, ctx->cub_bytes, ctx->scratch_bytes, ctx->Mcap, ctx->out_cols, ctx->cap};
+         ctx->d_Mind, ctx->d_m_val, ctx->d_res, ctx->d_work, ctx->d_Mval, ctx->d_tie, ctx->d_scratch,
+         ctx->tie_bytes, ctx->scratch_bytes, ctx->Mcap, ctx->out_cols, ctx->cap};
     ctx->d_counter = (int*)take(64 * sizeof(int));
-    ctx->d_queues = (int*)take((2 * kMaxBins + 1) * n * sizeof(int));
+    ctx->d_queues = (int*)take(kQueues * n * sizeof(int));
     ctx->d_m_len = (int*)take(n * sizeof(int));
     ctx->d_m_idx = (int*)take(n * cap * sizeof(int));
     ctx->d_m_val = (double*)take(n * cap * sizeof(double));
@@ -1866,8 +1865,6 @@ extern "C" int mspai_build_noalloc(mspai_ctx* ctx, const mspai_opts* opts, int* 
     ctx->d_status = (int*)take(n * sizeof(int));
     ctx->d_tie = take(tie);
     ctx->tie_bytes = tie;
-    ctx->d_cub = take(cub);
-    ctx->cub_bytes = cub;
     ctx->d_scratch = ctx->d_noalloc + off;
     ctx->scratch_bytes = kNoAllocBytes - off;
     ctx->d_work = nullptr;
@@ -1890,8 +1887,6 @@ extern "C" int mspai_build_noalloc(mspai_ctx* ctx, const mspai_opts* opts, int* 
     ctx->d_status = sv.status;
     ctx->d_tie = sv.tie;
     ctx->tie_bytes = sv.tie_bytes;
-    ctx->d_cub = sv.cub;
-    ctx->cub_bytes = sv.cub_bytes;
     ctx->d_scratch = sv.scr;
     ctx->scratch_bytes = sv.scr_bytes;
     ctx->d_work = sv.work;
