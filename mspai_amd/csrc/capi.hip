@@ -296,11 +296,8 @@ struct mspai_ctx {
     int* d_cache_status = nullptr;
     double* d_cache_data = nullptr;
     int tuned_table[2] = {-1, -1};  // autotuner's choice for this matrix (binning == 2), FP64 and mixed
-    int last_table = 0;
     int last_nbins = 0;
     unsigned long long first_end = 0;  // end of the first launch when the host looked at its counters (else 0)
-    bool last_mixed = false;
-    int last_binning = 1;
     bool last_counters = false;  // the last build stored per-column work counters
     long long nnzB = 0;
     int last_routed[8] = {0};
@@ -842,7 +839,7 @@ static int ensure_outputs(mspai_ctx* ctx, int cap)
     ctx->cap = cap;
     ctx->out_cols = n;
     ctx->Mcap = n * cap;
-    /* scan workspace for the compaction */
+    /* scan workspace of block builds */
     size_t need = 0;
     hipcub::DeviceScan::InclusiveSum(nullptr, need, ctx->d_m_len, ctx->d_Mptr + 1, (int)n, ctx->stream);
     need = std::max<size_t>(need, kNumWork * sizeof(double));
@@ -925,12 +922,11 @@ static ScratchLayout make_layout(int capJ, size_t capI, size_t capU, size_t capS
     /* register bins convert A(I,J) to FP32 as they load it: aq32 holds R only */
     const bool regbin = register_bin(group, (int)capI, capJ);
     /* the mixed builds' 64-lane LDS bins factor the Gram matrix instead of
-     * an FP32 copy of A(I,J) (not the adjoint, whose solve is the QR's) */
-    const bool gram = (needs & kNeedMixed) && !(needs & kNeedBackward) && group == 64 && !regbin;
+     * an FP32 copy of A(I,J) */
+    const bool gram = (needs & kNeedMixed) && group == 64 && !regbin;
     L.gram = gram;
     L.ldq = regbin ? capJ : (gram ? kGramLd : (int)capI);
     if (needs & kNeedMixed) L.aq32 = take((size_t)L.ldq * (gram ? kGramLd : capJ) * 4);
-    if (needs & kNeedBackward) L.rq = take((size_t)capJ * capJ * 8);
     if (needs & kNeedA0) {
         L.a0 = take(capI * capJ * 8);
         L.keep_a0 = 1;
@@ -938,8 +934,9 @@ static ScratchLayout make_layout(int capJ, size_t capI, size_t capU, size_t capS
     /* the FP32 right-hand side of the LDS QR and the vectors of its
      * refinement, and the adjoint's vectors (the register QR and its
      * refinement keep theirs in registers) */
-    if ((needs & kNeedBackward) || ((needs & kNeedMixed) && !regbin)) {
-        L.bq32 = take(capB * 4);
+    const bool refined = (needs & kNeedMixed) && !regbin;
+    if (refined) L.bq32 = take(capB * 4);
+    if (refined || (needs & kNeedBackward)) {
         L.g = take((size_t)capJ * 8);
         L.y = take((size_t)capJ * 8);
         L.z = take((size_t)capJ * 8);
@@ -1136,8 +1133,8 @@ static std::vector<Bin> bin_layouts(const mspai_ctx* ctx, int cap, int maxnew, b
         size_t capI = std::min<size_t>(G.capI, e.I);
         size_t capU = adaptive ? std::min<size_t>(G.capU, e.U) : 1;
         size_t capSort = std::min<size_t>(G.capSort, e.sort);
-        /* a mixed chain's FP64 bin: FP64 layout (the mixed build, not its adjoint) */
-        const int fp64 = (needs & kNeedMixed) && !(needs & kNeedBackward) && ((table.fp64mask >> t) & 1);
+        /* a mixed chain's FP64 bin: FP64 layout */
+        const int fp64 = (needs & kNeedMixed) && ((table.fp64mask >> t) & 1);
         const int bneeds = fp64 ? (needs & ~kNeedMixed) : needs;
         /* ties of scores across the cut are ordered in the generic kernel only */
         ScratchLayout L = make_layout(capJ, capI, capU, capSort, maxnew, 1, bneeds, false, e.group,
@@ -1658,7 +1655,6 @@ extern "C" int mspai_build(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* 
     const bool given = given_pattern_build(ctx, opts);
     if (given) {
         bins = static_wide_bins(ctx, cap, G, needs & ~kNeedMixed, opts->precision == 1);
-        ctx->last_table = table_for(ctx, opts);
     } else if (opts->binning && !ctx->d_up_ptr) {  // an upper pattern runs unbinned
         int t = table_for(ctx, opts);
         bins = bin_layouts(ctx, cap, opts->maxnew, adaptive, G, kTables[t], needs);
@@ -1667,7 +1663,6 @@ extern "C" int mspai_build(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* 
         fbins = (needs & kNeedMixed) ? bin_layouts(ctx, cap, opts->maxnew, adaptive, G, kTables[t],
                                                    needs & ~kNeedMixed)
                                      : bins;
-        ctx->last_table = t;
     }
     int gwaves = 0;
     if ((rc = prepare_generic(ctx, G, &gwaves))) return rc;
@@ -1775,9 +1770,7 @@ extern "C" int mspai_build(mspai_ctx* ctx, const mspai_opts* opts, mspai_stats* 
     ctx->nnzM = last;
     ctx->pattern_nnz = last;
     ctx->m_csr_ok = false;
-    ctx->last_mixed = mixed;
     ctx->mixed_fp64_last = mixed ? ctx->h_counter[62] : -1;
-    ctx->last_binning = opts->binning;
     ctx->last_counters = opts->counters != 0;
     if (stats) {
         std::memset(stats, 0, sizeof(*stats));

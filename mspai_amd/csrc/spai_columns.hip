@@ -65,7 +65,6 @@ struct WaveScratch {
     int* segoff;   // first flat entry of column J[t]; segoff[|J|] = total
     int* sid;      // flat entry -> position t in J
     double* wsum;  // the column's work counters
-    double* rq;    // adjoint: R of the register QR (capJ x capJ)
     double* a0;    // untouched copy of A(I,J), or nullptr
     unsigned* htab;  // row -> position hash of the candidate scores: always in LDS
     int hslots;      // its slots (a power of two)
@@ -105,7 +104,6 @@ __device__ __forceinline__ WaveScratch wave_scratch(char* ws, char* tie, const S
     s.segoff = (int*)(ws + L.segoff);
     s.sid = (int*)(ws + L.sid);
     s.wsum = (double*)(ws + L.wsum);
-    s.rq = (double*)(ws + L.rq);
     s.a0 = L.keep_a0 ? (double*)(ws + L.a0) : nullptr;
     s.htab = nullptr;  // set by the kernel (LDS)
     s.hslots = 0;
@@ -1166,7 +1164,7 @@ __device__ __forceinline__ double row_pick(const double (&a)[NMAX], int j)
  * holds the right-hand side; a reflector is applied to four slots at a time
  * so that their reductions interleave (slots outside (i, n) and b keep their
  * values). */
-template <int G, int NMAX, bool kROut = false>
+template <int G, int NMAX>
 __device__ __forceinline__ int ls_solve_regs(const ScratchLayout& L, const WaveScratch& s, int m, int n)
 {
     using Gr = Group<G>;
@@ -1234,16 +1232,6 @@ __device__ __forceinline__ int ls_solve_regs(const ScratchLayout& L, const WaveS
             zero_diag |= lane == i && rii == 0.0;
         }
     }
-    if (kROut) {
-        /* the adjoint's normal-equation solves need R, not x: R_iK (i <= K)
-         * to s.rq, column-major with leading dimension capJ */
-#pragma unroll
-        for (int K = 0; K < NMAX; ++K)
-            if (K < n && lane <= K) s.rq[K * L.capJ + lane] = a[K];
-        __syncthreads();
-        if (m < n) return COL_UNDERDET;
-        return Gr::ballot(zero_diag) != 0ull ? COL_SINGULAR : 0;
-    }
     double b = a[NMAX];
     int st = 0;
     if (m < n) {
@@ -1291,7 +1279,7 @@ __device__ __forceinline__ double rowgroup_sum_rt(F first, F2 next)
 /* NS column slots per lane (|J| <= 4 NS); slot NS holds b.  RT rows per
  * lane and slot: 4 (|I| <= 64) or 8 (|I| <= 128: rows q + 16 t, t = 0..7;
  * row r + 64 continues the chain of row r, as in the 64-lane order). */
-template <bool kROut, int NS = 8, int RT = 4>
+template <int NS = 8, int RT = 4>
 __device__ __forceinline__ int ls_solve_rows64(const ScratchLayout& L, const WaveScratch& s, int m, int n)
 {
     static_assert(RT == 4 || RT == 8, "rows per lane");
@@ -1377,18 +1365,6 @@ __device__ __forceinline__ int ls_solve_rows64(const ScratchLayout& L, const Wav
             }
             zero_diag |= c == ci && q == qi && rii == 0.0;
         }
-    }
-    if (kROut) {
-#pragma unroll
-        for (int sl = 0; sl < NS; ++sl)
-#pragma unroll
-            for (int t = 0; t < RT; ++t) {
-                const int j = c + 4 * sl, r = q + 16 * t;
-                if (j < n && r <= j) s.rq[j * L.capJ + r] = a[sl][t];
-            }
-        __syncthreads();
-        if (m < n) return COL_UNDERDET;
-        return __ballot(zero_diag) != 0ull ? COL_SINGULAR : 0;
     }
     int st = 0;
     if (m < n) {
@@ -2637,9 +2613,9 @@ __device__ __forceinline__ int solve_column(const BuildArgs& a, const ScratchLay
              * stored block and factor back from HBM): -cs serves the other
              * solves; both give the same bits */
             if constexpr (kRows128)
-                st |= ls_solve_rows64<false, NMAX / 4, 8>(L, s, m, n);
+                st |= ls_solve_rows64<NMAX / 4, 8>(L, s, m, n);
             else if constexpr (G == kWave && (NMAX == 32 || NMAX == 16))
-                st |= ls_solve_rows64<false, NMAX / 4>(L, s, m, n);
+                st |= ls_solve_rows64<NMAX / 4>(L, s, m, n);
             else
                 st |= ls_solve_regs<G, (NMAX > 0 ? NMAX : 4)>(L, s, m, n);
             dense = true;

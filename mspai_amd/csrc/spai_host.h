@@ -14,8 +14,8 @@ namespace mspai {
  * `group` lanes (16, 32 or 64), L.per_wave bytes of LDS per group; columns
  * that do not fit go to a.overflow.  mode 0: FP64 build; 1: FP32 QR + FP64
  * refinement, columns whose selection margins are too small go to
- * a.fallback; 2/3: the adjoint in FP64 / mixed; 4: FP64 build with the
- * dense QR update (-qr 2).  Without a queue (nullptr): columns
+ * a.fallback; 2: the adjoint (64-lane bins); 4: FP64 build with the dense QR
+ * update (-qr 2).  Without a queue (nullptr): columns
  * 0..a.nqueue, none seen by an earlier launch of the build. */
 void launch_binned(const BuildArgs& a, const ScratchLayout& L, int group, int mode, const int* queue,
                    const int* nqueue, int* head, int nwaves, hipStream_t stream, int wcap = 0);
