@@ -101,7 +101,6 @@ struct BuildArgs {
     double epsilon;
     int maxnew, ns, use_mean;
     int cap;                // capacity of one output column
-    int refine;             // precision 1: one refinement step in the workgroup kernel and in the adjoint's 64-lane bin
     int direct;             // static build: column k's outputs at p_ptr[k] (M has the start pattern) instead of k*cap
     int nqueue;             // columns 0..nqueue of a launch without a queue
     unsigned long long* stamp;  // start time of this launch
@@ -138,6 +137,7 @@ struct BuildArgs {
                             // decisions at the mean, at the maxnew cut, at epsilon, nnz of M)
     char* scratch;          // per-wave HBM working sets of the generic kernel
     char* tie_scratch;      // per-group HBM tie-path buffers of the LDS bins
+    int refine;             // precision 1: one refinement step in the workgroup kernel and in the adjoint's 64-lane bin
 };
 
 /* Block SPAI (-bs != 1): the block matrix, its patterns and the outputs.
