@@ -13,7 +13,7 @@ Prints one JSON line.  `value` is the columns/s of the mixed-precision build
 the size-binned against the unbinned (generic kernel only) FP64 build, the
 MSPAI probing workload (3D Laplacian 64^3, rho = 100) with its adjoint, and
 the block SPAI build.  `roofline` refers to the dominant column-kernel launch
-of the mixed build (HIP events on the library's stream around every launch);
+of the mixed build (by the kernels' own time stamps);
 `cpu_baseline` times the CPU FP64 restatement of the reference on this host.
 `--workload` selects another workload as the main line (profiling runs).
 """

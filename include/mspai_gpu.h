@@ -64,7 +64,7 @@ void mspai_default_opts(mspai_opts* o);
 
 /* Timing and counters of the last build. */
 typedef struct {
-    double build_ms;        /* device time of the whole build (HIP events) */
+    double build_ms;        /* device time of the whole build (time stamps of its kernels; block SPAI: HIP events) */
     double solve_ms;        /* device time of the column kernels only */
     long long nnz;          /* nnz of M */
     int ncols;
@@ -181,8 +181,10 @@ int mspai_result_values_device(mspai_ctx* ctx, double* d_out);
  * r = b - C(I,J) m, R^T R lambda = g, dL/dC(i,j) = r_i lambda_j -
  * (C lambda)_i m_j, dL/db = C lambda, with the QR recomputed in FP64 (when
  * opts->precision is 1 lambda takes one refinement step in columns of |J| <=
- * 40, |I| <= 128).  No counterpart in the reference (it has no derivatives); MSPAI probing weights rho enter through
- * C's and B's probe rows, so dL/drho follows from gC and gB by the chain rule.
+ * 40, |I| <= 128); degenerate columns have no gradient.  No counterpart in
+ * the reference (it has no derivatives); MSPAI probing weights rho enter
+ * through C's and B's probe rows, so dL/drho follows from gC and gB by the
+ * chain rule.
  * Accumulation into gC uses atomics, so its last bits depend on timing.
  */
 int mspai_backward(mspai_ctx* ctx, const mspai_opts* opts, const double* d_gM, double* d_gC, double* d_gB,
@@ -209,8 +211,9 @@ typedef struct {
 int mspai_autotune(mspai_ctx* ctx, const mspai_opts* opts, int repeats, mspai_tune_report* report);
 
 /* Sets the bin table that builds of `precision` (0 FP64, 1 mixed) with
- * opts->binning == 2 use (adaptive ones: see mspai_autotune), as the autotuner would (no counterpart in the
- * reference: for tests and for callers that tune once and store the choice).
+ * opts->binning == 2 use (adaptive ones, see mspai_autotune), as the
+ * autotuner would (no counterpart in the reference: for tests and for callers
+ * that tune once and store the choice).
  * `name` (32 bytes, may be NULL) receives the table's name, `ntables` (may be
  * NULL) the number of tables; table < 0 only reports that number.  Mixed
  * builds need a table with size bins (MSPAI_ERR_UNSUPPORTED otherwise). */
@@ -227,10 +230,10 @@ int mspai_work_totals(mspai_ctx* ctx, double* totals);
  * Per-launch profile of the last build or adjoint (no counterpart in the
  * reference): for every column-kernel launch in order, its name (precision,
  * size bin, lane-group width and |J|/|I| capacities, or the generic kernel),
- * its device time from HIP events on the library's stream, and -- after a
- * build with opts->counters set, else -1 -- the number of columns it
- * finished, the sums of their 8 work counters (as mspai_work_totals) and of
- * their near-margin decisions: FP64 selection decisions whose margin is at
+ * its device time from the kernels' own time stamps (to the next launch's
+ * start), and -- after a build with opts->counters set, else -1 -- the number
+ * of columns it finished, the sums of their 8 work counters (as
+ * mspai_work_totals) and of their near-margin decisions: FP64 selection decisions whose margin is at
  * most 1e-12 relative, so that another operation order could decide them
  * the other way (near[0]: a score against the mean threshold; near[1]: the
  * cut after the maxnew-th score, ties across it included; near[2]: ||r||

@@ -270,8 +270,8 @@ class Builder:
         return w
 
     def launch_stats(self):
-        """Per column-kernel launch of the last build: name, device ms (HIP
-        events), and with counters on the columns it finished, their work
+        """Per column-kernel launch of the last build: name, device ms (by
+        the kernels' time stamps), and with counters on the columns it finished, their work
         counter sums and near-margin decision counts (else -1)."""
         buf = (LaunchStat * 16)()
         n = C.c_int()

@@ -39,10 +39,9 @@ constexpr int kStampEnd = kMaxLaunch + 3;
 constexpr int kNumStamps = kMaxLaunch + 4;
 
 /* Device scratch of mspai_build_noalloc (queues, counters, output slots,
- * per-column results, tie buffers, the scan workspace and the generic
- * kernel's working sets of one build), a static array so that the call
- * allocates nothing.  Each device the library runs on holds its own copy
- * until the process ends.  In host code `scratch` only names the symbol:
+ * per-column results, tie buffers and the generic kernel's working sets of
+ * one build), a static array so that the call allocates nothing.  Each device
+ * the library runs on holds its own copy until the process ends.  In host code `scratch` only names the symbol:
  * its device address comes from hipGetSymbolAddress, once per device (at
  * mspai_ctx_create), and that address is what the kernels receive.  Calls
  * on one device share the array: calls that overlap on one GPU race. */
@@ -68,7 +67,8 @@ void dfree(T*& p)
  * nullptr: not wanted), kValueLanes lanes per column.  Every stored entry
  * finds its column in its row by a binary search, a chain of dependent reads:
  * latency-bound, so the lanes of a column search together -- 3.1 M entries in
- * rows of 12: 200 us with one thread per column, 33 us so. */
+ * rows of 12: 109 us for both parts (profiles/kernel_times_cases.md), 17 and
+ * 198 us as two launches with one thread per column. */
 constexpr int kValueLanes = 8;
 
 __global__ __launch_bounds__(256) void column_values_kernel(DevCsc A, double* ajn, int norm_blocks, const int* rp_ptr,

@@ -18,7 +18,7 @@
  * Rows and slots that a step no longer touches are skipped at compile time
  * (rows) or by a uniform branch (slots).  On P(A^2) of the 3D
  * variable-coefficient operator (|J| <= 25, |I| <= 63, n = 2,097,152) an FP64
- * build takes 27.9 ms, 4.9 K VALU instructions per column; with four rows per
+ * build takes 27.5 ms, 5.0 K VALU instructions per column; with four rows per
  * lane and four lane moves per dot product (the adaptive builds' register QR)
  * it took 64.1 ms and 13.3 K.  Values and gradient of the 48^3 operator: 8.2
  * -> 3.4 ms; of MSPAI probing on the 64^3 Laplacian at precision 1: 3.3 ->

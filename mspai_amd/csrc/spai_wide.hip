@@ -1,6 +1,7 @@
 /*
- * FP64 adaptive column kernel for wide columns: one column of M per workgroup
- * of eight waves, |J| <= 40, |I| <= 384.
+ * FP64 column kernel for wide columns (adaptive builds, and static ones past the
+ * given-pattern kernels): one column of M per workgroup of eight waves,
+ * |J| <= 40, |I| <= 384.
  *
  * What bounds it: few columns reach these sizes (954 of the 262,144-column
  * random band), so the launch takes as long as its slowest column: six steps
